@@ -165,6 +165,7 @@ struct uocr_hip_moe_layer {
     float scaling = 1.0f, rms_eps = 1e-6f;
     int device = 0;
     uint16_t* router_t = nullptr;
+    uint16_t* router_m = nullptr;  // bf16 router in the prefill router's operand order
     float* router_f32 = nullptr;  // [hidden/4][64][4] (decode router)
     float* rms_weight = nullptr;
     uint8_t* gate = nullptr;   // [Ev][inter x hidden] tile layout
@@ -210,7 +211,7 @@ namespace {
 
 void free_layer(uocr_hip_moe_layer* L) {
     if (!L) return;
-    void* ptrs[] = {L->router_t, L->router_f32, L->rms_weight, L->gate,   L->up,   L->down, L->gate_s,
+    void* ptrs[] = {L->router_t, L->router_m, L->router_f32, L->rms_weight, L->gate,   L->up,   L->down, L->gate_s,
                     L->up_s,     L->down_s,     L->gate_z,     L->up_z,   L->down_z, L->sync, L->down_skt, L->down_zkt, L->sw,
                     L->sgate,    L->sup,        L->sdown,      L->egate,  L->eup,    L->edown};
     for (void* p : ptrs)
@@ -421,7 +422,7 @@ int uocr_hip_moe_layer_create(const uocr_hip_layer_desc* d, uocr_hip_moe_layer**
     const int H = d->hidden, I = d->inter, E = d->n_experts;
     if (H <= 0 || I <= 0 || H % kTileK || I % kTileK)
         return fail(UOCR_HIP_EINVAL, "hidden and inter must be positive multiples of 128");
-    if (router_smem_bytes(H) > 150 * 1024 || H > 1792 || I > 1792)
+    if (H > 1792 || I > 1792)
         return fail(UOCR_HIP_EUNSUPPORTED, "hidden/inter above 1792 are not supported by this build");
     if (E <= 0 || E > 64) return fail(UOCR_HIP_EINVAL, "n_experts must be in [1, 64]");
     if (d->top_k <= 0 || d->top_k > kMaxTopK || d->top_k > E)
@@ -623,6 +624,16 @@ int uocr_hip_moe_layer_create(const uocr_hip_layer_desc* d, uocr_hip_moe_layer**
                 for (int i = 0; i < 8; ++i) rt[((size_t)c8 * E + e) * 8 + i] = d->router_bf16[(size_t)e * H + c8 * 8 + i];
     }
 
+    // and in the prefill router's MFMA operand order [H/32][4][64][8]: element
+    // s of (32-column step c32, k-slice g, expert e) is column c32 * 32 + 4 s + g
+    std::vector<uint16_t> rm;
+    if (!d->router_f32) {
+        rm.assign((size_t)H * 64, 0);
+        for (int e = 0; e < E; ++e)
+            for (int c = 0; c < H; ++c)
+                rm[((size_t)(c / 32 * 4 + c % 4) * 64 + e) * 8 + c % 32 / 4] = d->router_bf16[(size_t)e * H + c];
+    }
+
     // and as f32 [H/4][64][4] for the decode router (experts padded to 64 with
     // zeros, so a 64-column chunk is one contiguous 16 KiB block)
     std::vector<float> rf((size_t)H * 64, 0.0f);
@@ -696,6 +707,7 @@ int uocr_hip_moe_layer_create(const uocr_hip_layer_desc* d, uocr_hip_moe_layer**
     };
     const bool int4 = Ev > 0;
     if ((!rt.empty() && (rc = up_copy((void**)&L->router_t, rt.data(), rt.size() * 2, "router"))) ||
+        (!rm.empty() && (rc = up_copy((void**)&L->router_m, rm.data(), rm.size() * 2, "router (operand order)"))) ||
         (rc = up_copy((void**)&L->router_f32, rf.data(), rf.size() * 4, "router f32")) ||
         (int4 && (rc = up_copy((void**)&L->gate, hg.data(), hg.size(), "gate"))) ||
         (int4 && (rc = up_copy((void**)&L->up, hu.data(), hu.size(), "up"))) ||
@@ -935,8 +947,7 @@ int uocr_hip_moe_layer_forward(const uocr_hip_moe_layer* L, const void* x, int x
             ra.top_k = L->top_k;
             ra.rms_weight = L->rms_weight;
             ra.rms_eps = L->rms_eps;
-            ra.router_t = L->router_t;
-    ra.router_f32 = L->router_f32;
+            ra.router_m = L->router_m;
             ra.norm_topk_prob = L->norm_topk_prob;
             ra.scoring_sigmoid = L->scoring_sigmoid;
             ra.scaling = L->scaling;
@@ -965,8 +976,7 @@ int uocr_hip_moe_layer_forward(const uocr_hip_moe_layer* L, const void* x, int x
     ra.top_k = L->top_k;
     ra.rms_weight = L->rms_weight;
     ra.rms_eps = L->rms_eps;
-    ra.router_t = L->router_t;
-    ra.router_f32 = L->router_f32;
+    ra.router_m = L->router_m;
     ra.norm_topk_prob = L->norm_topk_prob;
     ra.scoring_sigmoid = L->scoring_sigmoid;
     ra.scaling = L->scaling;

@@ -39,8 +39,7 @@ struct RouterArgs {
     int seq, hidden, n_experts, top_k;
     const float* rms_weight;  // optional [hidden]
     float rms_eps;
-    const uint16_t* router_t; // router W as [hidden/8][n_experts][8] bf16
-    const float* router_f32;  // the same W as f32 [hidden/4][64][4] (experts padded to 64), or null
+    const uint16_t* router_m; // router W in MFMA operand order, bf16 [hidden/32][4][64][8] (experts padded to 64)
     int norm_topk_prob, scoring_sigmoid;
     float scaling;
     f16* x16;                 // out [seq, hidden] f16 expert input
@@ -192,7 +191,6 @@ bool decode_stream_ok(int hidden, int inter, int group);
 hipError_t launch_decode_stream(const DecodeArgs& a, hipStream_t st);
 
 hipError_t launch_router(const RouterArgs& a, bool x_is_bf16, hipStream_t st);
-size_t router_smem_bytes(int hidden);
 constexpr int kDecodeTileRows = 16;
 constexpr int kPrefillTileRows = 128;     // generic prefill kernel
 constexpr int kPrefillBigTileRows = 256;  // large-tile prefill kernel (K in {896, 1280})

@@ -452,286 +452,225 @@ __global__ __launch_bounds__(256) void group_place_kernel(GroupArgs g) {
 }
 
 // ---------------------------------------------------------------------------
-// Router: one wave per token, lane e owns expert e (E <= 64); a workgroup of W
-// waves routes W tokens (W = 4 for small batches, so the FMA chains of
-// different tokens run on different SIMDs and CUs; W = 16 for large batches,
-// so each streamed weight chunk serves 16 tokens). The router matrix
-// ([H/8][E][8] bf16) streams through LDS in double-buffered 128-column chunks,
-// so every lane's FMA chain reads its weights from LDS instead of issuing one
-// dependent global load per 8 columns.
+// Router for a bf16 router matrix (E <= 64): 16 tokens per workgroup of 16
+// waves, the logits on v_mfma_f32_16x16x4_f32.
+//
+// The f32 MFMA accumulates its k-slices in ascending order with one rounding
+// per term and keeps denormals, so a chain of them gives the bits of the
+// reference's sequential fmaf chain. Waves 0..3 own 16 experts each and run one chain for
+// all 16 tokens: 32.3 cycles per 4 columns, against
+// 4 x (17..23) cycles per column and token for one lane per expert. The
+// RMSNorm's sum of squares (each product rounded, then added in column order)
+// is the same chain with ones as the other operand: fma(x * x, 1, sum).
+//   * x rows in LDS as f32, every 16 columns transposed 4 x 4 so that one
+//     16-byte read holds a lane's operand of four consecutive MFMAs; rows are
+//     padded by 16 bytes (16 tokens then cover all 64 banks);
+//   * router_m holds the weights in the order of the other operand (8 MFMAs
+//     per 16-byte load), read from L2 ten loads ahead;
+//   * 16 waves, because scoring and top-k take one wave per token.
+// Bound by the chain's latency (1280 columns: 320 MFMAs, 10.4k cycles alone,
+// 14k measured; with the RMSNorm a second chain), the token rows' arrival and
+// the top-k (7k cycles). Measured against one lane per expert and token
+// (rocprofv3): 1024 tokens 16.4 -> 13.0 us, 4096 tokens 34 -> 17.8, 1111 tokens
+// 30.8 -> 15.7, 283 tokens with the RMSNorm 39 -> 21.7.
 // ---------------------------------------------------------------------------
-constexpr int kChunkC8 = 16;  // 128 columns per chunk
+constexpr int kRouterTokens = 16;
+constexpr int kMaxRouterHidden = 1792;
+constexpr int kLogitStride = 68;  // floats per token of the logits in LDS
 
-__host__ __device__ constexpr size_t router_lds_bytes(int H, int waves) {
-    return (size_t)waves * H * 4          // xs
-           + 2ull * kChunkC8 * 64 * 16    // W chunks (E <= 64)
-           + (size_t)waves * 64 * 4;      // per-wave scores
+// LDS byte offset of column c (a multiple of 16) in a token row: 16 bytes of
+// padding per 64 columns, so that the staging writes (64 bytes apart per
+// lane) cover all banks too; rows are an odd number of 16-byte units
+__host__ __device__ constexpr int router_col_bytes(int c) { return c * 4 + c / 64 * 16; }
+__host__ __device__ constexpr int router_row_bytes(int H) { return router_col_bytes(H) + 16; }
+__host__ __device__ constexpr size_t router_lds_bytes(int H) {
+    return (size_t)kRouterTokens * router_row_bytes(H) + (size_t)kRouterTokens * kLogitStride * 4 +
+           (size_t)kRouterTokens * 64 * 4;
 }
 
-constexpr int kMaxChunks = 14;  // hidden <= 1792
-
-template <typename XT, bool RMS, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void router_kernel(RouterArgs a) {
+// HC: hidden as a compile-time constant (the k-loops are then unrolled and the
+// weights stay four 32-column steps ahead in registers); 0: a.hidden, one step
+template <typename XT, bool RMS, int HC>
+__global__ __launch_bounds__(kRouterTokens * 64) void router_kernel(RouterArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    constexpr int NT = WAVES * 64;
-    constexpr int UPT = kChunkC8 * 64 / NT;  // 16-byte chunk units per thread (E <= 64)
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, tid = threadIdx.x;
-    const int H = a.hidden, E = a.n_experts, K = a.top_k;
-    float* xs = reinterpret_cast<float*>(smem) + (size_t)wave * H;
-    u32x4* wb = reinterpret_cast<u32x4*>(smem + (size_t)WAVES * H * 4);
-    float* scr = reinterpret_cast<float*>(wb + 2 * kChunkC8 * 64) + wave * 64;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int H = HC ? HC : a.hidden, E = a.n_experts, K = a.top_k;
+    const int rowb = router_row_bytes(H), n_steps = H / 32;
+    float* logits = reinterpret_cast<float*>(smem + (size_t)kRouterTokens * rowb);
+    float* scr = logits + kRouterTokens * kLogitStride + wave * 64;
     __shared__ uint64_t etab[32];
+    __shared__ float inv_s[kRouterTokens];
     if (threadIdx.x < 32) etab[threadIdx.x] = uocr_exp2_tab[threadIdx.x];
-    const int t = blockIdx.x * WAVES + wave;
+    const int t = blockIdx.x * kRouterTokens + wave;
     const bool live = t < a.seq;
-    const XT* x = static_cast<const XT*>(a.x);
-    const int chunk_units = kChunkC8 * E;
-    const u32x4* wsrc = reinterpret_cast<const u32x4*>(a.router_t);
-    const int n_chunks = H / (kChunkC8 * 8);
+    const XT* x = static_cast<const XT*>(a.x) + (size_t)min(t, a.seq - 1) * H;
+    const int m16 = lane & 15, g = lane >> 4;
 
-    // every router-weight load of this thread, all chunks, issued at once
-    u32x4 wreg[kMaxChunks][UPT];
+    // waves 0..3: the weights of 16 experts. 32-column step i: 8 bf16 of
+    // expert 16 * wave + m16, MFMA s of the step taking column 4 s + g
+    constexpr int RING = HC ? 10 : 1;
+    u32x4 wreg[RING];
+    const u32x4* wsrc = reinterpret_cast<const u32x4*>(a.router_m) + g * 64 + wave * 16 + m16;
+    if (wave < 4) {
 #pragma unroll
-    for (int ch = 0; ch < kMaxChunks; ++ch)
-#pragma unroll
-        for (int j = 0; j < UPT; ++j) {
-            const int u = tid + j * NT;
-            if (ch < n_chunks && u < chunk_units) wreg[ch][j] = wsrc[(size_t)ch * chunk_units + u];
-        }
-    // this wave's token row, as f32
-    for (int c = lane * 8; c < H; c += 64 * 8) {
-        float v[8];
-        if (live) {
-            load8_f32<XT>(x + (size_t)t * H + c, v);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = 0.0f;
-        }
-        *reinterpret_cast<f32x4*>(xs + c) = f32x4{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<f32x4*>(xs + c + 4) = f32x4{v[4], v[5], v[6], v[7]};
-    }
-#pragma unroll
-    for (int j = 0; j < UPT; ++j)
-        if (tid + j * NT < chunk_units) wb[tid + j * NT] = wreg[0][j];
-    __syncthreads();
-
-    if constexpr (RMS) {
-        if (lane == 0) {
-            float ss = 0.0f;
-            for (int c = 0; c < H; c += 4) {
-                const f32x4 v = *reinterpret_cast<const f32x4*>(xs + c);
-                // the reference build rounds each x*x and sums in order (H % 4 == 0 here)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) ss = __fadd_rn(ss, __fmul_rn(v[i], v[i]));
-            }
-            scr[0] = __fdiv_rn(1.0f, sqrt_rn(__fadd_rn(__fdiv_rn(ss, (float)H), a.rms_eps)));
-        }
-        __syncthreads();
-        const float inv = scr[0];
-        for (int c = lane; c < H; c += 64) xs[c] = __fmul_rn(__fmul_rn(xs[c], inv), a.rms_weight[c]);
-        __syncthreads();
+        for (int i = 0; i < RING; ++i) wreg[i] = wsrc[i * 256];
     }
 
-    if (live) {
-        for (int c = lane * 8; c < H; c += 64 * 8) {
-            const f32x4 p = *reinterpret_cast<const f32x4*>(xs + c);
-            const f32x4 q = *reinterpret_cast<const f32x4*>(xs + c + 4);
-            f16x8 h = {(f16)p[0], (f16)p[1], (f16)p[2], (f16)p[3], (f16)q[0], (f16)q[1], (f16)q[2], (f16)q[3]};
-            *reinterpret_cast<f16x8*>(a.x16 + (size_t)t * H + c) = h;
-        }
-    }
-
-    // logits: lane e runs the sequential fmaf chain over all H columns
-    float acc = 0.0f;
-    if constexpr (!RMS && WAVES == 16) {
-        // The token row is the same for every lane of the wave: it comes in
-        // through scalar loads (16 dwords per block, the next block requested
-        // while this one is consumed), so LDS serves only the weight reads.
-        constexpr int DW = 2 * (int)sizeof(XT);  // dwords per 8 columns
-        constexpr int BC = 16 / DW;               // 8-column steps per block
-        constexpr int NB = kChunkC8 / BC;         // blocks per chunk
-        const int n_blocks = n_chunks * NB;
-        const int tu = min(__builtin_amdgcn_readfirstlane(t), a.seq - 1);
-        const uint64_t row = (uint64_t)(x + (size_t)tu * H);
-        auto block_load = [&](int b, u32x16& q) {
-            const uint64_t ad = row + (uint64_t)min(b, n_blocks - 1) * 64u;
-            asm volatile("s_load_dwordx16 %0, %1, 0x0" : "=s"(q) : "s"(ad) : "memory");
-        };
-        u32x16 c0;
-        block_load(0, c0);
+    // this wave's token row: 16 columns per lane and step. store_x16 writes
+    // the experts' f16 input
+    auto store_x16 = [&](int c, const float* v) {
+        f16x8 h[2];
 #pragma unroll
-        for (int ch = 0; ch < kMaxChunks; ++ch) {
-            if (ch < n_chunks) {
-                const u32x4* cur = wb + (ch & 1) * kChunkC8 * 64;
-#pragma unroll
-                for (int bl = 0; bl < NB; ++bl) {
-                    // (acc ties the previous block's chain to this point, so
-                    // the loads are not all hoisted to the chunk's start)
-                    asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(c0), "+v"(acc)::"memory");
-                    u32x16 n0;
-                    block_load(ch * NB + bl + 1, n0);
-#pragma unroll
-                    for (int i = 0; i < BC; ++i) {
-                        const u32x4 wv = cur[(bl * BC + i) * E + lane];
-                        float xv[8];
-#pragma unroll
-                        for (int k = 0; k < DW; ++k) {
-                            const uint32_t d = c0[DW * i + k];
-                            if constexpr (sizeof(XT) == 2) {
-                                xv[2 * k] = __uint_as_float(d << 16);
-                                xv[2 * k + 1] = __uint_as_float(d & 0xffff0000u);
-                            } else {
-                                xv[k] = __uint_as_float(d);
-                            }
-                        }
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            acc = fmaf(xv[2 * k], __uint_as_float(wv[k] << 16), acc);
-                            acc = fmaf(xv[2 * k + 1], __uint_as_float(wv[k] & 0xffff0000u), acc);
-                        }
-                    }
-                    c0 = n0;
-                }
-                if (ch + 1 < kMaxChunks && ch + 1 < n_chunks) {
-#pragma unroll
-                    for (int j = 0; j < UPT; ++j)
-                        if (tid + j * NT < chunk_units)
-                            wb[((ch + 1) & 1) * kChunkC8 * 64 + tid + j * NT] = wreg[ch + 1][j];
-                }
-                __syncthreads();
-            }
-        }
-        // the last block's (clamped, repeated) loads must land before exit
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(c0)::"memory");
-    } else
-#pragma unroll
-    for (int ch = 0; ch < kMaxChunks; ++ch) {
-        if (ch < n_chunks) {
-            const u32x4* cur = wb + (ch & 1) * kChunkC8 * 64;
-            if (lane < E) {
-#pragma unroll 4
-                for (int c8 = 0; c8 < kChunkC8; ++c8) {
-                    const u32x4 wv = cur[c8 * E + lane];
-                    const float* xp = xs + (ch * kChunkC8 + c8) * 8;
-                    const f32x4 xa = *reinterpret_cast<const f32x4*>(xp);
-                    const f32x4 xb = *reinterpret_cast<const f32x4*>(xp + 4);
-                    acc = fmaf(xa[0], __uint_as_float(wv[0] << 16), acc);
-                    acc = fmaf(xa[1], __uint_as_float(wv[0] & 0xffff0000u), acc);
-                    acc = fmaf(xa[2], __uint_as_float(wv[1] << 16), acc);
-                    acc = fmaf(xa[3], __uint_as_float(wv[1] & 0xffff0000u), acc);
-                    acc = fmaf(xb[0], __uint_as_float(wv[2] << 16), acc);
-                    acc = fmaf(xb[1], __uint_as_float(wv[2] & 0xffff0000u), acc);
-                    acc = fmaf(xb[2], __uint_as_float(wv[3] << 16), acc);
-                    acc = fmaf(xb[3], __uint_as_float(wv[3] & 0xffff0000u), acc);
-                }
-            }
-            if (ch + 1 < kMaxChunks && ch + 1 < n_chunks) {
-#pragma unroll
-                for (int j = 0; j < UPT; ++j)
-                    if (tid + j * NT < chunk_units) wb[((ch + 1) & 1) * kChunkC8 * 64 + tid + j * NT] = wreg[ch + 1][j];
-            }
-            __syncthreads();
-        }
-    }
-
-    // scoring and greedy top-k by the wave alone (no workgroup barrier)
-    const WaveTopk pick = wave_topk(acc, E, K, a.scoring_sigmoid, a.norm_topk_prob, a.scaling, scr, etab);
-    if (live && lane < K) a.weights[(size_t)t * K + lane] = pick.w;
-    if (live && pick.rank < K) a.ids[(size_t)t * K + pick.rank] = lane;
-}
-
-
-// Router without the RMSNorm prologue for fewer than 4096 tokens: one token
-// per wave, one wave per SIMD, where a wave issues one VALU op every several
-// cycles whatever the dependences. The weights therefore come from the f32
-// copy of the router ([H/4][64][4]: a 128-column chunk is one contiguous
-// 32 KiB block), so a column costs one FMA and no widening; the chunks stream
-// through LDS from a register ring as in router_kernel.
-constexpr int kF32ChunkUnits = kChunkC8 * 2 * 64;  // 16-byte units per 128-column chunk
-
-__host__ __device__ constexpr size_t router_f32w_lds_bytes(int H) {
-    return (size_t)4 * H * 4                     // xs
-           + 2ull * kF32ChunkUnits * 16         // W chunks
-           + (size_t)4 * 64 * 4;                // per-wave scores
-}
-
-template <typename XT>
-__global__ __launch_bounds__(256) void router_f32w_kernel(RouterArgs a) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    constexpr int WAVES = 4, NT = 256;
-    constexpr int UPT = kF32ChunkUnits / NT;  // 8
-    constexpr int RING = 3;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, tid = threadIdx.x;
-    const int H = a.hidden, E = a.n_experts, K = a.top_k;
-    float* xs = reinterpret_cast<float*>(smem) + (size_t)wave * H;
-    f32x4* wb = reinterpret_cast<f32x4*>(smem + (size_t)WAVES * H * 4);
-    float* scr = reinterpret_cast<float*>(wb + 2 * kF32ChunkUnits) + wave * 64;
-    __shared__ uint64_t etab[32];
-    if (threadIdx.x < 32) etab[threadIdx.x] = uocr_exp2_tab[threadIdx.x];
-    const int t = blockIdx.x * WAVES + wave;
-    const bool live = t < a.seq;
-    const XT* x = static_cast<const XT*>(a.x);
-    const f32x4* wsrc = reinterpret_cast<const f32x4*>(a.router_f32);
-    const int n_chunks = H / (kChunkC8 * 8);
-
-    f32x4 wreg[RING][UPT];
-    auto issue_chunk = [&](int ch) {
-#pragma unroll
-        for (int j = 0; j < UPT; ++j)
-            if (ch < n_chunks) wreg[ch % RING][j] = wsrc[(size_t)ch * kF32ChunkUnits + tid + j * NT];
+        for (int i = 0; i < 16; ++i) h[i >> 3][i & 7] = (f16)v[i];
+        f16* d = a.x16 + (size_t)t * H + c;
+        reinterpret_cast<f16x8*>(d)[0] = h[0];
+        reinterpret_cast<f16x8*>(d)[1] = h[1];
     };
+    // (RMS: the row stays in registers and LDS first holds the rounded squares)
+    unsigned char* xrow = smem + (size_t)wave * rowb;
+    auto put = [&](int c, const float* v) {
 #pragma unroll
-    for (int ch = 0; ch < RING; ++ch) issue_chunk(ch);
-    // this wave's token row, as f32 (and as f16 for the experts)
-    for (int c = lane * 8; c < H; c += 64 * 8) {
-        float v[8];
-        if (live) {
-            load8_f32<XT>(x + (size_t)t * H + c, v);
-        } else {
+        for (int q = 0; q < 4; ++q)
+            *reinterpret_cast<f32x4*>(xrow + router_col_bytes(c) + q * 16) = f32x4{v[q], v[4 + q], v[8 + q], v[12 + q]};
+    };
+    constexpr int NV = (kMaxRouterHidden + 1023) / 1024;
+    float v[NV][16];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = 0.0f;
+    for (int j = 0; j < NV; ++j) {
+        const int c = lane * 16 + j * 1024;
+        if (c < H) {
+            load8_f32<XT>(x + c, v[j]);
+            load8_f32<XT>(x + c + 8, v[j] + 8);
         }
-        *reinterpret_cast<f32x4*>(xs + c) = f32x4{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<f32x4*>(xs + c + 4) = f32x4{v[4], v[5], v[6], v[7]};
-        if (live)
-            *reinterpret_cast<f16x8*>(a.x16 + (size_t)t * H + c) =
-                f16x8{(f16)v[0], (f16)v[1], (f16)v[2], (f16)v[3], (f16)v[4], (f16)v[5], (f16)v[6], (f16)v[7]};
     }
 #pragma unroll
-    for (int j = 0; j < UPT; ++j) wb[tid + j * NT] = wreg[0][j];
-    if (RING < kMaxChunks) issue_chunk(RING);
+    for (int j = 0; j < NV; ++j) {
+        const int c = lane * 16 + j * 1024;
+        if (c < H) {
+            float sq[16];
+            if constexpr (RMS) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sq[i] = __fmul_rn(v[j][i], v[j][i]);
+            }
+            put(c, RMS ? sq : v[j]);
+            if (!RMS && live) store_x16(c, v[j]);
+        }
+    }
     __syncthreads();
 
-    // logits: lane e runs the sequential fmaf chain over all H columns (lanes
-    // >= E run the zero padding)
-    float acc = 0.0f;
+    // operand reads: token m16, k-slice g, the 8 MFMAs of 32-column step i
+    const unsigned char* xop = smem + (size_t)m16 * rowb + g * 16;
+    auto read_x = [&](int i, f32x4* v) {
+        const int c = (i < n_steps ? i : n_steps - 1) * 32;  // (past the end: the last step again)
+        v[0] = *reinterpret_cast<const f32x4*>(xop + router_col_bytes(c));
+        v[1] = *reinterpret_cast<const f32x4*>(xop + router_col_bytes(c) + 64);
+    };
+    // One chain step per MFMA, accumulating in place (asm: the compiler would
+    // rotate the accumulator through other registers, which costs the chain
+    // wait states). A VALU op between two MFMAs of a chain costs it 13 cycles,
+    // eight of them after eight MFMAs 5.7 per MFMA, a ds_read 3 (measured on
+    // one wave: 32.3 cycles per MFMA alone), so a step's other work comes in
+    // one piece. s_nop 1 covers a VALU write of an operand, which the hazard
+    // recognizer does not see in asm, and chain_end() the wait states before
+    // the result is read.
+    auto mac = [](f32x4& acc, float p, float q) {
+        asm volatile("s_nop 1\n\tv_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+v"(acc) : "v"(p), "v"(q));
+    };
+    auto chain_begin = [](f32x4& acc) {
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("s_nop 7" : "+v"(acc));
+    };
+    auto chain_end = [](f32x4& acc) { asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc)); };
+    if constexpr (RMS) {
+        if (wave == 0) {
+            f32x4 ss, cur[2], nx[2];
+            read_x(0, cur);
+            const float one = 1.0f;
+            chain_begin(ss);
+            auto step = [&](int i, f32x4* u, f32x4* next) {
+                read_x(i + 1, next);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ch = 0; ch < kMaxChunks; ++ch) {
-        if (ch < n_chunks) {
-            const f32x4* cur = wb + (ch & 1) * kF32ChunkUnits;
-            const float* xc = xs + ch * kChunkC8 * 8;
-            // 32 steps of 4 columns; the LDS reads run 6 steps ahead of the
-            // FMAs with explicit lgkmcnt waits (the compiler's schedule waits
-            // on every read pair or hoists every read of the chunk)
-            const uint32_t w_addr = lds_addr(cur) + lane * 16;
-            const uint32_t x_addr = lds_addr(xc);
-            asm volatile(UOCR_RCHUNK(UOCR_RMAC_FMA)
-                : [acc] "+v"(acc)
-                : [w] "v"(w_addr), [x] "v"(x_addr)
-                : "v64", "v65", "v66", "v67", "v68", "v69", "v70", "v71", "v72", "v73", "v74", "v75", "v76", "v77",
-                  "v78", "v79", "v80", "v81", "v82", "v83", "v84", "v85", "v86", "v87", "v88", "v89", "v90", "v91",
-                  "v92", "v93", "v94", "v95", "v96", "v97", "v98", "v99", "v100", "v101", "v102", "v103", "v104",
-                  "v105", "v106", "v107", "v108", "v109", "v110", "v111", "memory");
-            if (ch + 1 < kMaxChunks && ch + 1 < n_chunks) {
-#pragma unroll
-                for (int j = 0; j < UPT; ++j) wb[((ch + 1) & 1) * kF32ChunkUnits + tid + j * NT] = wreg[(ch + 1) % RING][j];
-                if (ch + 1 + RING < kMaxChunks) issue_chunk(ch + 1 + RING);
+                for (int s = 0; s < 8; ++s) mac(ss, u[s >> 2][s & 3], one);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            for (int i = 0; i < n_steps; i += 2) {  // (H % 128 == 0)
+                step(i, cur, nx);
+                step(i + 1, nx, cur);
             }
-            __syncthreads();
+            chain_end(ss);
+            // lane holds the sums of tokens 4 g + r (the same in every column m16)
+            float s = ss[0];
+#pragma unroll
+            for (int r = 1; r < 4; ++r) s = (m16 & 3) == r ? ss[r] : s;
+            if (m16 < 4)
+                inv_s[4 * g + m16] = __fdiv_rn(1.0f, sqrt_rn(__fadd_rn(__fdiv_rn(s, (float)H), a.rms_eps)));
         }
+        __syncthreads();
+        const float inv = inv_s[wave];
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int c = lane * 16 + j * 1024;
+            if (c < H) {
+                float w[16];
+                load8_f32<float>(a.rms_weight + c, w);
+                load8_f32<float>(a.rms_weight + c + 8, w + 8);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) v[j][i] = __fmul_rn(__fmul_rn(v[j][i], inv), w[i]);
+                put(c, v[j]);
+                if (live) store_x16(c, v[j]);
+            }
+        }
+        __syncthreads();
     }
 
-    const WaveTopk pick = wave_topk(acc, E, K, a.scoring_sigmoid, a.norm_topk_prob, a.scaling, scr, etab);
+    if (wave < 4) {
+        f32x4 acc, xa[2], xb[2];
+        float wa[8], wb[8];
+        auto widen = [](const u32x4& w, float* o) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s) o[s] = __uint_as_float(s & 1 ? w[s >> 1] & 0xffff0000u : w[s >> 1] << 16);
+        };
+        // rows: experts, columns: tokens. Step i: x of step i + 1 is requested,
+        // the MFMAs run, then the weights of step i + 1 are widened and those
+        // of step i + RING requested
+        read_x(0, xa);
+        widen(wreg[0], wa);
+        chain_begin(acc);
+        auto step = [&](int i, const float* wc, const f32x4* xc, float* wn, f32x4* xn, const u32x4& w, u32x4& refill) {
+            read_x(i + 1, xn);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) mac(acc, wc[s], xc[s >> 2][s & 3]);
+            __builtin_amdgcn_sched_barrier(0);
+            widen(w, wn);
+            if (i + RING < n_steps) refill = wsrc[(size_t)(i + RING) * 256];
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if constexpr (HC > 0) {
+#pragma unroll
+            for (int i = 0; i < HC / 32; i += 2) {
+                step(i, wa, xa, wb, xb, wreg[(i + 1) % RING], wreg[i % RING]);
+                step(i + 1, wb, xb, wa, xa, wreg[(i + 2) % RING], wreg[(i + 1) % RING]);
+            }
+        } else {
+            u32x4 none;
+            for (int i = 0; i < n_steps; i += 2) {
+                const u32x4 w1 = wsrc[(size_t)(i + 1) * 256];
+                step(i, wa, xa, wb, xb, w1, none);
+                const u32x4 w2 = wsrc[(size_t)min(i + 2, n_steps - 1) * 256];
+                step(i + 1, wb, xb, wa, xa, w2, none);
+            }
+        }
+        chain_end(acc);
+        // lane holds experts 16 * wave + 4 g + r of token m16
+        *reinterpret_cast<f32x4*>(logits + m16 * kLogitStride + wave * 16 + 4 * g) = acc;
+    }
+    __syncthreads();
+
+    // scoring and greedy top-k of one token per wave
+    const WaveTopk pick = wave_topk(logits[wave * kLogitStride + lane], E, K, a.scoring_sigmoid, a.norm_topk_prob,
+                                    a.scaling, scr, etab);
     if (live && lane < K) a.weights[(size_t)t * K + lane] = pick.w;
     if (live && pick.rank < K) a.ids[(size_t)t * K + pick.rank] = lane;
 }
@@ -802,46 +741,28 @@ __global__ __launch_bounds__(256) void router_from_logits_kernel(RouterArgs a, c
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
-size_t router_smem_bytes(int hidden) { return router_lds_bytes(hidden, 16); }
-
-template <typename XT, bool RMS, int WAVES>
-static hipError_t launch_router_t(const RouterArgs& a, hipStream_t st) {
+template <typename XT, bool RMS, int HC>
+static hipError_t launch_router_h(const RouterArgs& a, hipStream_t st) {
     // > 64 KiB of dynamic LDS: raise the limit once per kernel
-    static hipError_t attr = hipFuncSetAttribute((const void*)router_kernel<XT, RMS, WAVES>,
+    static hipError_t attr = hipFuncSetAttribute((const void*)router_kernel<XT, RMS, HC>,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
     if (attr != hipSuccess) return attr;
-    const dim3 grid((a.seq + WAVES - 1) / WAVES);
-    launch_k((router_kernel<XT, RMS, WAVES>), grid, dim3(WAVES * 64), router_lds_bytes(a.hidden, WAVES),
-                       st, a);
-    return hipGetLastError();
-}
-
-template <typename XT>
-static hipError_t launch_router_f32w(const RouterArgs& a, hipStream_t st) {
-    static hipError_t attr = hipFuncSetAttribute((const void*)router_f32w_kernel<XT>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
-    if (attr != hipSuccess) return attr;
-    launch_k((router_f32w_kernel<XT>), dim3((a.seq + 3) / 4), dim3(256), router_f32w_lds_bytes(a.hidden), st, a);
+    launch_k((router_kernel<XT, RMS, HC>), dim3((a.seq + kRouterTokens - 1) / kRouterTokens),
+             dim3(kRouterTokens * 64), router_lds_bytes(a.hidden), st, a);
     return hipGetLastError();
 }
 
 template <typename XT, bool RMS>
-static hipError_t launch_router_w(const RouterArgs& a, hipStream_t st) {
-    if constexpr (!RMS) {
-        if (a.seq < 4096 && a.router_f32) return launch_router_f32w<XT>(a, st);
-    }
-    // 4 tokens per workgroup spread the FMA chains over the CUs; once that
-    // gives 4+ workgroups per CU (4096 tokens on 256 CUs), 16 tokens per
-    // workgroup amortise the router-weight stream
-    return a.seq >= 4096 ? launch_router_t<XT, RMS, 16>(a, st) : launch_router_t<XT, RMS, 4>(a, st);
+static hipError_t launch_router_t(const RouterArgs& a, hipStream_t st) {
+    return a.hidden == 1280 ? launch_router_h<XT, RMS, 1280>(a, st) : launch_router_h<XT, RMS, 0>(a, st);
 }
 
 hipError_t launch_router(const RouterArgs& a, bool x_is_bf16, hipStream_t st) {
-    if (a.n_experts > 64 || a.hidden > kMaxChunks * kChunkC8 * 8 || a.hidden % (kChunkC8 * 8))
+    if (a.n_experts > 64 || a.hidden > kMaxRouterHidden || a.hidden % 128 || a.seq <= 0 || !a.router_m)
         return hipErrorInvalidValue;
     const bool rms = a.rms_weight != nullptr;
-    if (x_is_bf16) return rms ? launch_router_w<uint16_t, true>(a, st) : launch_router_w<uint16_t, false>(a, st);
-    return rms ? launch_router_w<float, true>(a, st) : launch_router_w<float, false>(a, st);
+    if (x_is_bf16) return rms ? launch_router_t<uint16_t, true>(a, st) : launch_router_t<uint16_t, false>(a, st);
+    return rms ? launch_router_t<float, true>(a, st) : launch_router_t<float, false>(a, st);
 }
 
 hipError_t launch_router_from_logits(const RouterArgs& a, const float* logits, hipStream_t st) {
