@@ -1,0 +1,103 @@
+"""The query-tiled attention kernel (head_dim 64 or 128, 98304 or more (row,
+head, key) triples) against the oracle: tile and key-block edges, rows of several requests
+in one tile, tiles left to the row workers, grouped heads, empty rows.
+
+Both kernels hold everything in f32; the tolerance is that of the row kernel's
+tests (1e-4 absolute on outputs of order 1)."""
+import numpy as np
+import pytest
+
+import oracle as O
+from test_gpu_rswa import TOL, dev_f32, dev_i32, lib, ok, ptr, rand
+
+pytestmark = pytest.mark.gpu
+
+
+def _torch():
+    import torch
+    return torch
+
+
+@pytest.mark.parametrize("hd,kv_heads,heads", [(128, 10, 10), (64, 2, 8), (128, 2, 6)])
+@pytest.mark.parametrize("lens", [
+    [260],                       # one request, a ragged last tile
+    [31, 33, 64, 1, 129],        # tile boundaries inside and between requests
+    [3] * 40 + [70],             # short requests: tiles of many slots
+])
+def test_ragged_tiles(dev, hd, kv_heads, heads, lens):
+    torch = _torch()
+    print(f"[rswa tile] ragged hd={hd} heads={heads}/{kv_heads} lens={lens[:6]}", flush=True)
+    rng = np.random.default_rng(hd + heads + len(lens))
+    cap, st, n = max(max(lens) + 5, 200), kv_heads * hd, len(lens)
+    K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
+    slots = rng.permutation(n).astype(np.int32)
+    d_slots = np.concatenate([[s] * m for s, m in zip(slots, lens)]).astype(np.int32)
+    d_pos = np.concatenate([np.arange(m) for m in lens]).astype(np.int32)
+    total = len(d_pos)
+    assert total * heads >= 512 and total * heads * cap >= 98304
+    q = rand(rng, total, heads, hd)
+    out = torch.full((q.size,), float("nan"), dtype=torch.float32, device=dev)
+    ok(lib().uocr_hip_rswa_attention_ragged(ptr(dev_f32(q, dev)), ptr(dev_f32(K, dev)), ptr(dev_f32(V, dev)),
+                                            ptr(dev_i32(d_slots, dev)), ptr(dev_i32(d_pos, dev)), total, cap, heads,
+                                            kv_heads, hd, ptr(out), None))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().reshape(total, heads * hd)
+    t0 = 0
+    for s, m in zip(slots, lens):
+        want = O.rswa_attention(q[t0:t0 + m], K[s], V[s], m, 0, heads, kv_heads, hd, True).reshape(m, -1)
+        assert np.abs(got[t0:t0 + m] - want).max() <= TOL, (s, m)
+        t0 += m
+
+
+def test_ragged_rows_in_any_order(dev):
+    """Rows of long caches, every row another slot or position (a tile costs
+    more than its rows): the row workers; and a tile that mixes both."""
+    torch = _torch()
+    rng = np.random.default_rng(5)
+    kv_heads = heads = 10
+    hd, n, cap = 128, 40, 300
+    K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
+    d_slots = np.concatenate([rng.permutation(n), [7] * 50]).astype(np.int32)
+    d_pos = np.concatenate([rng.integers(0, cap, n), rng.permutation(cap)[:50]]).astype(np.int32)
+    total = len(d_pos)
+    q = rand(rng, total, heads, hd)
+    out = torch.full((q.size,), float("nan"), dtype=torch.float32, device=dev)
+    print("[rswa tile] rows in any order", flush=True)
+    ok(lib().uocr_hip_rswa_attention_ragged(ptr(dev_f32(q, dev)), ptr(dev_f32(K, dev)), ptr(dev_f32(V, dev)),
+                                            ptr(dev_i32(d_slots, dev)), ptr(dev_i32(d_pos, dev)), total, cap, heads,
+                                            kv_heads, hd, ptr(out), None))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().reshape(total, -1)
+    for t in range(total):
+        L = int(d_pos[t]) + 1
+        want = O.rswa_attention(q[t:t + 1], K[d_slots[t]], V[d_slots[t]], L, 0, heads, kv_heads, hd, False).ravel()
+        assert np.abs(got[t] - want).max() <= TOL, t
+
+
+@pytest.mark.parametrize("seq,q_start,kv_len,causal", [(64, 936, 1000, 1), (129, 0, 129, 1), (300, 0, 33, 0),
+                                                       (180, -120, 60, 1), (210, 0, 50, 1)])
+def test_one_cache_tiles(dev, seq, q_start, kv_len, causal):
+    """The query-block entry points with the length on the host and on the
+    device; rows before the first key (q_start < 0) have no keys and give 0."""
+    torch = _torch()
+    rng = np.random.default_rng(seq + kv_len)
+    kv_heads = heads = 10
+    hd = 128
+    assert seq * heads * kv_len >= 98304
+    print(f"[rswa tile] one cache seq={seq} q_start={q_start} kv_len={kv_len} causal={causal}", flush=True)
+    K, V = rand(rng, kv_len, kv_heads, hd), rand(rng, kv_len, kv_heads, hd)
+    q = rand(rng, seq, heads, hd)
+    lo = max(0, -q_start) if causal else 0
+    want = np.zeros((seq, heads * hd), np.float32)
+    want[lo:] = O.rswa_attention(q[lo:], K, V, kv_len, q_start + lo, heads, kv_heads, hd, causal).reshape(seq - lo, -1)
+    kc, vc, dq = dev_f32(K, dev), dev_f32(V, dev), dev_f32(q, dev)
+    for devlen in (False, True):
+        out = torch.full((q.size,), float("nan"), dtype=torch.float32, device=dev)
+        if devlen:
+            ok(lib().uocr_hip_rswa_attention_devlen(ptr(dq), ptr(kc), ptr(vc), ptr(dev_i32([kv_len], dev)), seq,
+                                                    q_start, heads, kv_heads, hd, causal, ptr(out), None))
+        else:
+            ok(lib().uocr_hip_rswa_attention(ptr(dq), ptr(kc), ptr(vc), kv_len, seq, q_start, heads, kv_heads, hd,
+                                             causal, ptr(out), None))
+        torch.cuda.synchronize()
+        assert np.abs(out.cpu().numpy().reshape(seq, -1) - want).max() <= TOL, devlen

@@ -6,7 +6,7 @@
 // prefill ("reference tokens"), rows P..P+W-1 a ring of the last W decoded
 // tokens.
 //
-// Attention: one workgroup per (query row, head), 8 waves splitting the keys.
+// Attention, row kernel: one workgroup per (query row, head), 8 waves splitting the keys.
 // A wave takes groups of 8 consecutive keys (groups w, w + 8, ...): lane
 // (j, p) = (lane / 8, lane % 8) holds key j's dims 4p + 32i .. + 3 (i < HDP / 32)
 // of K and V (each load: the 8 lanes of a key read one contiguous 128-byte run),
@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <initializer_list>
 #include <mutex>
 #include <string>
@@ -53,11 +54,19 @@ struct RswaArgs {
 // one partial record: m, l, (pad), then o[head_dim]
 constexpr int kRswaRec = 256 + 4;
 
-template <int HDP>
-__global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
+// LDS of one row's wave results
+template <int HDP, int WAVES>
+struct RowLds {
+    float m[WAVES], l[WAVES];
+    __attribute__((aligned(16))) float acc[WAVES][HDP];
+};
+
+// One (query row, head) by a workgroup of WAVES waves; keys split over
+// n_chunks calls (chunk = chunk).
+template <int HDP, int WAVES>
+__device__ __forceinline__ void row_attention(const RswaArgs& a, int row, int head, int chunk, RowLds<HDP, WAVES>& s) {
     constexpr int D = HDP / 8;  // dims per lane
     constexpr int NV = D / 4;   // float4 per lane per row
-    const int row = blockIdx.x, head = blockIdx.y;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int j = lane >> 3, p = lane & 7;
     const int hd = a.head_dim, stride = a.kv_heads * hd;
@@ -96,7 +105,7 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
     int kbeg = 0, kend = limit;
     if (a.n_chunks > 1) {
         const int cs = ((limit + a.n_chunks - 1) / a.n_chunks + 7) & ~7;
-        kbeg = min(limit, (int)blockIdx.z * cs);
+        kbeg = min(limit, chunk * cs);
         kend = min(limit, kbeg + cs);
     }
     const int n_groups = (kend - kbeg + 7) / 8;
@@ -128,13 +137,13 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
         part += __shfl_xor(part, 2, 64);
         part += __shfl_xor(part, 4, 64);
         const bool valid = kbeg + g * 8 + j < kend;
-        const float s = valid ? part * a.scale : -INFINITY;
-        float mg = fmaxf(s, __shfl_xor(s, 8, 64));
+        const float sc = valid ? part * a.scale : -INFINITY;
+        float mg = fmaxf(sc, __shfl_xor(sc, 8, 64));
         mg = fmaxf(mg, __shfl_xor(mg, 16, 64));
         mg = fmaxf(mg, __shfl_xor(mg, 32, 64));
         const float m_new = fmaxf(m, mg);  // finite: key 0 of the group is valid
         const float alpha = __builtin_amdgcn_exp2f((m - m_new) * kLog2e);
-        const float beta = valid ? __builtin_amdgcn_exp2f((s - m_new) * kLog2e) : 0.0f;
+        const float beta = valid ? __builtin_amdgcn_exp2f((sc - m_new) * kLog2e) : 0.0f;
         float bs = beta + __shfl_xor(beta, 8, 64);
         bs += __shfl_xor(bs, 16, 64);
         bs += __shfl_xor(bs, 32, 64);
@@ -147,7 +156,7 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
     };
     // groups wave, wave + 8, ...; two groups' loads in flight beyond the one in
     // use (three register buffers in rotation), one for head_dim > 128
-    constexpr int GS = kRswaWaves;
+    constexpr int GS = WAVES;
     int g = wave;
     if constexpr (HDP <= 128) {
         if (g < n_groups) {
@@ -190,8 +199,9 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
             x += __shfl_xor(x, 32, 64);
             acc[i][c] = x;
         }
-    __shared__ float wm[kRswaWaves], wl[kRswaWaves];
-    __shared__ __attribute__((aligned(16))) float wacc[kRswaWaves][HDP];
+    auto& wm = s.m;
+    auto& wl = s.l;
+    auto& wacc = s.acc;
     if (lane < 8) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) *reinterpret_cast<f32x4*>(&wacc[wave][dim_of(i)]) = acc[i];
@@ -202,28 +212,28 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
     }
     __syncthreads();
     // combine the waves (a wave without keys has m = -inf and weight 0)
-    float* rec = a.n_chunks > 1 ? a.part + (((size_t)row * a.heads + head) * a.n_chunks + blockIdx.z) * kRswaRec
+    float* rec = a.n_chunks > 1 ? a.part + (((size_t)row * a.heads + head) * a.n_chunks + chunk) * kRswaRec
                                 : nullptr;
     if (rec && tid == 0) {
         float M = -INFINITY, L = 0.0f;
 #pragma unroll
-        for (int w = 0; w < kRswaWaves; ++w) M = fmaxf(M, wm[w]);
+        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, wm[w]);
         if (M != -INFINITY) {
 #pragma unroll
-            for (int w = 0; w < kRswaWaves; ++w)
+            for (int w = 0; w < WAVES; ++w)
                 L = fmaf(wl[w], wm[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((wm[w] - M) * kLog2e), L);
         }
         rec[0] = M;
         rec[1] = L;
     }
-    for (int d = tid; d < hd; d += kRswaWaves * 64) {
+    for (int d = tid; d < hd; d += WAVES * 64) {
         float M = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < kRswaWaves; ++w) M = fmaxf(M, wm[w]);
+        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, wm[w]);
         float L = 0.0f, o = 0.0f;
         if (M != -INFINITY) {
 #pragma unroll
-            for (int w = 0; w < kRswaWaves; ++w) {
+            for (int w = 0; w < WAVES; ++w) {
                 const float f = wm[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((wm[w] - M) * kLog2e);
                 L = fmaf(wl[w], f, L);
                 o = fmaf(wacc[w][d], f, o);
@@ -233,6 +243,377 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
             rec[4 + d] = o;  // unnormalised, relative to this chunk's max
         else
             a.out[qoff + d] = L > 0.0f ? o / L : 0.0f;
+    }
+}
+
+template <int HDP>
+__global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
+    __shared__ RowLds<HDP, kRswaWaves> s;
+    row_attention<HDP, kRswaWaves>(a, blockIdx.x, blockIdx.y, blockIdx.z, s);
+}
+
+// ---------------------------------------------------------------------------
+// Query-tiled attention (prefill): a workgroup of 4 waves takes 32 consecutive
+// query rows of one head on v_mfma_f32_32x32x2_f32; the waves split the keys
+// in blocks of 32 (block w, w + 4, ...) with an online softmax per wave and
+// are combined at the end, as in the row kernel. f32 throughout.
+//   * S^T = K Q^T: lane (i, h) = (lane % 32, lane / 32) holds key i's operand and
+//     query i's, step s of unit pair j taking dims 8 j + 4 h + s; so one 16-byte read
+//     serves four MFMAs. K blocks come by DMA into LDS, their 16-byte units
+//     permuted per key (unit u at u ^ key) so that the reads of 16 keys
+//     cover all banks;
+//   * D holds keys 8 (r / 4) + 4 h + r % 4 of query i, which is the operand
+//     layout of O^T = V^T P^T with the keys taken in that order: the
+//     probabilities never leave their lane. V rows come straight from global
+//     memory, 16 bytes (dims 4 i .. + 3) per lane: dim-block b's MFMA takes
+//     dims 4 i + b.
+// The rows of a tile may belong to several requests (slots): one pass over the
+// keys per distinct slot, rows of other slots masked. Where that costs more
+// than walking the rows one by one (a key block of a pass costs about four
+// row-blocks of the row kernel: 9 against 2.2 ns on the whole chip), the tile
+// is left to row workers, extra workgroups at the grid's end.
+// Bound by the f32 MFMA rate (154 TFLOP/s on a large product; 35 us of the
+// call below), the start of a workgroup (9k cycles to its first scores) and the grid's end.
+// Measured (rocprofv3) at 4 requests of 358..1000 rows, 10 heads of 128: 711 us
+// row by row, 123 us tiled; error against 64 bits 1.41e-7 both ways (one
+// chain per score and per output is 7% faster and 3.2e-7 off). Not kept: 8
+// waves per workgroup, one per CU (the start is then exposed: 160 us); all 16
+// V rows in flight with Q in registers (spills).
+// ---------------------------------------------------------------------------
+constexpr int kTileQ = 32;        // query rows per tile
+constexpr int kTileWaves = 4;     // two workgroups per CU (head_dim 128: 80 KiB of LDS each)
+constexpr int kTileSort = kTileWaves * 64;  // tiles that a call orders by their keys (one per thread)
+static_assert(kTileSort <= 256, "a tile's index has 8 bits of its sort key");
+constexpr int kTileCost = 4;      // row-blocks that a tile's key block costs
+constexpr int kRowWorkers = 512;  // at most
+constexpr long long kTileMinWork = 98304;
+
+// slot and key limit (rows attended, 0 past the end) of query row t
+__device__ __forceinline__ void row_limit(const RswaArgs& a, int rows, int t, int& slot, int& limit) {
+    slot = -1;
+    limit = 0;
+    if (t >= rows) return;
+    if (a.mode == 3) {
+        slot = a.d_slots[t];
+        limit = a.d_pos[t] + 1;
+    } else {
+        const int kv_len = a.mode == 1 ? *a.d_len : a.kv_len;
+        slot = 0;
+        limit = a.causal ? min(kv_len, a.q_start + t + 1) : kv_len;
+    }
+    limit = max(limit, 0);
+}
+
+__device__ __forceinline__ int half_max(int v) {  // over the 32 lanes of a half wave
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// whether a tile (lane l: row l % 32's slot and limit) runs as a tile;
+// wave-uniform. (Its buffer loads address up to 2 GiB of a request's cache.)
+__device__ __forceinline__ bool tile_size_ok(const RswaArgs& a, int limit) {
+    return (long long)limit * a.kv_heads * a.head_dim * 4 <= 0x7fffffffll;
+}
+__device__ __forceinline__ bool tile_pays(const RswaArgs& a, int slot, int limit) {
+    if (!tile_size_ok(a, half_max(limit))) return false;
+    int rows = (limit + 31) / 32, cost = 0;
+    for (int o = 16; o >= 1; o >>= 1) rows += __shfl_xor(rows, o, 64);
+    uint32_t left = (uint32_t)__ballot(limit > 0);
+    while (left) {
+        const int s = __shfl(slot, __builtin_ctz(left), 64);
+        const bool in = slot == s && limit > 0;
+        cost += (half_max(in ? limit : 0) + 31) / 32 * kTileCost;
+        left &= ~(uint32_t)__ballot(in);
+    }
+    return __builtin_amdgcn_readfirstlane(cost) <= __builtin_amdgcn_readfirstlane(rows);
+}
+// by one thread: false if the tile certainly runs as a tile (its runs of rows of
+// one slot, an upper bound of its passes, cost no more than its rows)
+__device__ __forceinline__ bool tile_may_not_pay(const RswaArgs& a, int rows, int tile) {
+    int slots[kTileQ], limits[kTileQ];  // every load in flight before the first use
+#pragma unroll
+    for (int r = 0; r < kTileQ; ++r) row_limit(a, rows, tile * kTileQ + r, slots[r], limits[r]);
+    int n = 0, cost = 0, run = 0, most = 0;
+#pragma unroll
+    for (int r = 0; r < kTileQ; ++r) {
+        const int blocks = (limits[r] + 31) / 32;
+        if (r > 0 && slots[r] != slots[r - 1]) {
+            cost += run;
+            run = 0;
+        }
+        run = max(run, blocks);
+        most = max(most, limits[r]);
+        n += blocks;
+    }
+    return !tile_size_ok(a, most) || (cost + run) * kTileCost > n;
+}
+
+__device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+
+template <int HD>
+struct TileLds {
+    __attribute__((aligned(16))) float k[kTileWaves][32 * HD];  // K blocks, then the waves' outputs
+    union {
+        __attribute__((aligned(16))) float q[32 * HD];
+        struct {  // once the last scores are done
+            float m[kTileWaves][32], l[kTileWaves][32];
+        };
+    };
+};
+
+template <int HD>
+__global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs a, int rows, int n_tiles, bool sort) {
+    constexpr int U = HD / 4;    // 16-byte units per row
+    constexpr int NB = HD / 32;  // dims per lane of V, dim-blocks of O
+    union Lds {
+        TileLds<HD> t;
+        RowLds<HD, kTileWaves> r;
+        struct {
+            int list[kTileSort], n_list;
+        };
+        struct {
+            __attribute__((aligned(16))) int pos[kTileSort];
+            int tile;
+        };
+    };
+    __shared__ Lds s;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (scalar: it is in the loads' scalar offsets)
+    const int i = lane & 31, h = lane >> 5;
+    int slot, limit;
+    if ((int)blockIdx.x >= n_tiles * a.heads) {  // row worker: the rows of the tiles that don't pay
+        const int w = blockIdx.x - n_tiles * a.heads, nw = gridDim.x - n_tiles * a.heads;
+        int& n_list = s.n_list;
+        for (int t0 = 0; t0 < n_tiles; t0 += kTileSort) {
+            if (tid == 0) n_list = 0;
+            __syncthreads();
+            if (t0 + tid < n_tiles && tile_may_not_pay(a, rows, t0 + tid)) s.list[atomicAdd(&n_list, 1)] = t0 + tid;
+            __syncthreads();
+            const int n_l = n_list, mine = tid < n_l ? s.list[tid] : 0;
+            __syncthreads();
+            for (int k = 0; k < n_l; ++k) {
+                if (tid == k) n_list = mine;
+                __syncthreads();
+                const int tile = n_list;
+                __syncthreads();  // (the rows' results take the list's place)
+                row_limit(a, rows, tile * kTileQ + i, slot, limit);
+                if (tile_pays(a, slot, limit)) continue;
+                const int n = min(kTileQ, rows - tile * kTileQ) * a.heads;
+                for (int j = w; j < n; j += nw) {
+                    row_attention<HD, kTileWaves>(a, tile * kTileQ + j / a.heads, j % a.heads, 0, s.r);
+                    __syncthreads();
+                }
+            }
+        }
+        return;
+    }
+    // The tiles with the most keys first, so that the grid's end is made of
+    // short ones (sort: more workgroups than the chip holds at once): the tile
+    // whose last row's position has rank blockIdx.x / heads (ties by index). Beyond kTileSort tiles: in reverse order.
+    const int rank = blockIdx.x / a.heads, head = blockIdx.x % a.heads;
+    int tile = n_tiles - 1 - rank;
+    if (a.mode == 3 && n_tiles <= kTileSort && sort) {
+        // (position, index) in one word: distinct whatever the positions
+        const int mine = tid < n_tiles
+                             ? (int)((uint32_t)a.d_pos[min(tid * kTileQ + kTileQ, rows) - 1] << 8 | (255 - tid))
+                             : INT_MIN;
+        s.pos[tid] = mine;
+        __syncthreads();
+        if (tid < n_tiles) {
+            int before = 0;
+#pragma unroll 4
+            for (int j = 0; j < n_tiles; j += 4) {
+                const int4 p = *reinterpret_cast<const int4*>(&s.pos[j]);
+                before += (p.x > mine) + (p.y > mine) + (p.z > mine) + (p.w > mine);
+            }
+            if (before == rank) s.tile = tid;
+        }
+        __syncthreads();
+        tile = __builtin_amdgcn_readfirstlane(s.tile);
+        __syncthreads();
+    }
+    row_limit(a, rows, tile * kTileQ + i, slot, limit);
+    if (!tile_pays(a, slot, limit)) return;
+    const int stride = a.kv_heads * HD;
+    const int kvh = head / (a.heads / a.kv_heads);
+    constexpr float kLog2e = 1.4426950408889634f;
+
+    // the query rows in LDS (registers are for O and V), units permuted as K's
+    for (int u = tid; u < 32 * U; u += kTileWaves * 64) {
+        const int r = u / U, c = u % U;
+        const float* qr = a.q + ((size_t)min(tile * kTileQ + r, rows - 1) * a.heads + head) * HD;
+        *reinterpret_cast<f32x4*>(&s.t.q[r * HD + (c ^ (r % U)) * 4]) = *reinterpret_cast<const f32x4*>(qr + 4 * c);
+    }
+    __syncthreads();
+    float m = -INFINITY, l = 0.0f;  // of query i, over this lane's keys (l) / the wave's (m)
+    f32x16 o[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) o[b] = f32x16{};
+
+    float* kbuf = s.t.k[wave];
+    uint32_t left = (uint32_t)__ballot(limit > 0);
+    while (left) {  // one pass per distinct slot
+        const int ps = __builtin_amdgcn_readfirstlane(__shfl(slot, __builtin_ctz(left), 64));
+        const bool in = slot == ps && limit > 0;
+        left &= ~(uint32_t)__ballot(in);
+        const int mylim = in ? limit : 0;
+        const int kend = __builtin_amdgcn_readfirstlane(half_max(mylim));
+        const size_t base = (a.mode == 3 ? (size_t)ps * a.batch_cap * stride : 0) + (size_t)kvh * HD;
+        // buffer loads: keys past kend are out of range and read as zeros
+        // (base + kvh * HD: the last key's row ends before the next key's)
+        const int bytes = ((kend - 1) * stride + HD) * 4, rowb = stride * 4;
+        const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.kc + base), 0, bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.vc + base), 0, bytes, 0x00020000);
+        const int nblk = (kend + 31) / 32;
+        // DMA n covers 64 / U keys, unit u of key k at u ^ (k % U)
+        // (the asm statements keep the 16 offsets from being hoisted out of the
+        // key loop, where they would spill)
+        const int kvo = (lane / U) * rowb;
+        int ku = ((lane % U) ^ (lane / U)) << 4;
+        auto load_k = [&](int blk) {
+            asm volatile("" : "+v"(ku));
+#pragma unroll
+            for (int n = 0; n < U / 2; ++n)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                    kr, (__attribute__((address_space(3))) void*)(kbuf + n * 256), 16,
+                    kvo + (ku ^ ((n * (64 / U)) % U << 4)), (blk * 32 + n * (64 / U)) * rowb, 0, 0);
+        };
+        const int vvo = 4 * h * rowb + NB * i * 4;
+        if (wave < nblk) load_k(wave);
+        for (int blk = wave; blk < nblk; blk += kTileWaves) {
+            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the K block has landed
+            __builtin_amdgcn_sched_barrier(0);
+            // V of this block: rows r < 8 in flight during the scores, the
+            // others during the softmax (all 16 at once would spill)
+            float v[2][8][NB];
+            auto load_v = [&](int half) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    const int so = (blk * 32 + 16 * half + 8 * (r >> 2) + (r & 3)) * rowb;
+                    if constexpr (NB == 4) {
+                        const f32x4 t = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, vvo, so, 0));
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) v[half][r][b] = t[b];
+                    } else {
+                        const u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(vr, vvo, so, 0));
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) v[half][r][b] = __uint_as_float(t[b]);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            load_v(0);
+            // K reads two unit pairs (8 MFMAs) ahead; the barriers keep the
+            // scheduler from hoisting all of them (64 registers)
+            // (short chains round less: two at a time, over quarters of the dims)
+            f32x16 st[2], sum16;
+            f32x4 kv[3], qv[3];
+            int ko = i * HD + ((h ^ (i % U)) << 2);
+            asm volatile("" : "+v"(ko));
+            auto read_k = [&](int j) {
+                kv[j % 3] = *reinterpret_cast<const f32x4*>(kbuf + (ko ^ (j << 3)));
+                qv[j % 3] = *reinterpret_cast<const f32x4*>(s.t.q + (ko ^ (j << 3)));
+            };
+            read_k(0);
+            read_k(1);
+#pragma unroll
+            for (int j = 0; j < U / 2; ++j) {
+                if (j + 2 < U / 2) read_k(j + 2);
+                if (j % (U / 8) == 0) st[0] = st[1] = f32x16{};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) st[c & 1] = mfma_f32(kv[j % 3][c], qv[j % 3][c], st[c & 1]);
+                if (j % (U / 8) == U / 8 - 1) {
+                    if (j < U / 8) sum16 = st[0] + st[1];
+                    else sum16 += st[0] + st[1];
+                    asm volatile("" : "+v"(sum16));  // added here (later, the chains would keep their registers)
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): K is in registers, the buffer is free
+            __builtin_amdgcn_sched_barrier(0);
+            load_v(1);
+            if (blk + kTileWaves < nblk) load_k(blk + kTileWaves);
+            __builtin_amdgcn_sched_barrier(0);
+            // online softmax of query i over this lane's 16 keys and its partner's
+            float p[16], mx = -INFINITY;
+            const int lim = mylim - blk * 32 - 4 * h;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                p[r] = 8 * (r >> 2) + (r & 3) < lim ? sum16[r] * a.scale : -INFINITY;
+                mx = fmaxf(mx, p[r]);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float mn = fmaxf(m, mx);
+            const float mref = mn == -INFINITY ? 0.0f : mn;
+            const float alpha = __builtin_amdgcn_exp2f((m - mref) * kLog2e);
+            float sum[4] = {};
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                p[r] = __builtin_amdgcn_exp2f((p[r] - mref) * kLog2e);
+                sum[r & 3] += p[r];
+            }
+            l = fmaf(l, alpha, (sum[0] + sum[1]) + (sum[2] + sum[3]));
+            m = mn;
+            // a block's keys are summed from zero in four chains of 8, then
+            // added (rounds less than one chain over all keys)
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    f32x16 ob[2] = {};
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int c = 0; c < 2; ++c)
+                            ob[c] = mfma_f32(v[half][4 * c + r][b], p[8 * half + 4 * c + r], ob[c]);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        o[b][r] = half ? o[b][r] + (ob[0][r] + ob[1][r]) : fmaf(o[b][r], alpha, ob[0][r] + ob[1][r]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        }
+    }
+    // combine the waves: each leaves its unnormalised rows [query][dim] in its
+    // own K buffer (unit permuted by the query), then every thread sums
+    l += __shfl_xor(l, 32, 64);
+    __syncthreads();  // the query rows' place takes m and l
+    if (h == 0) {
+        s.t.m[wave][i] = m;
+        s.t.l[wave][i] = l;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int rho = 8 * (r >> 2) + 4 * h + (r & 3);  // dims NB * rho .. + NB - 1
+        if constexpr (NB == 4) {
+            *reinterpret_cast<f32x4*>(kbuf + i * HD + (rho ^ i) * 4) = f32x4{o[0][r], o[1][r], o[2][r], o[3][r]};
+        } else {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) kbuf[i * HD + (rho ^ i) * NB + b] = o[b][r];
+        }
+    }
+    __syncthreads();
+    for (int u = tid; u < 32 * 32; u += kTileWaves * 64) {
+        const int qi = u / 32, rho = u % 32, row = tile * kTileQ + qi;
+        if (row >= rows) continue;
+        float M = -INFINITY, L = 0.0f, acc[NB] = {};
+#pragma unroll
+        for (int w = 0; w < kTileWaves; ++w) M = fmaxf(M, s.t.m[w][qi]);
+        if (M != -INFINITY) {
+#pragma unroll
+            for (int w = 0; w < kTileWaves; ++w) {
+                const float f = __builtin_amdgcn_exp2f((s.t.m[w][qi] - M) * kLog2e);
+                L = fmaf(s.t.l[w][qi], f, L);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) acc[b] = fmaf(s.t.k[w][qi * HD + (rho ^ qi) * NB + b], f, acc[b]);
+            }
+        }
+        float* op = a.out + ((size_t)row * a.heads + head) * HD + NB * rho;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) op[b] = L > 0.0f ? acc[b] / L : 0.0f;
     }
 }
 
@@ -370,7 +751,8 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
     float* part = nullptr;
     int cus = 0;
     const long long wgs = (long long)rows * a.heads;
-    if (wgs < 512 && rswa_device(&part, &cus) == 0) {
+    const bool known = rswa_device(&part, &cus) == 0;
+    if (wgs < 512 && known) {
         int n = (int)((2LL * cus + wgs - 1) / wgs);
         if (max_len > 0) n = std::min(n, max_len / 128);
         n = std::min(n, 8);
@@ -379,6 +761,22 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
             a.n_chunks = n;
             a.part = part;
         }
+    }
+    // One cache or ragged rows run query-tiled where the kernel is instantiated
+    // (head_dim 64 and 128), from kTileMinWork (row, head, key) triples, keys
+    // as far as the host knows them: below, the row kernel's shorter start
+    // wins (heads x rows x keys at head_dim 128, us against tiled: 600 x 60 13.1
+    // / 15.0, 970 x 60 15.6 / 19.2, 1630 x 60 23.6 / 24.1, 1300 x 130 23.7 / 17.6, 3000 x
+    // 300 57 / 26). Fewer than 512 pairs keep the key split above.
+    if (wgs >= 512 && a.mode != 2 && (a.head_dim == 64 || a.head_dim == 128) &&
+        wgs * (max_len > 0 ? max_len : 128) >= kTileMinWork) {
+        const int n_tiles = (rows + kTileQ - 1) / kTileQ;
+        const dim3 tgrid(n_tiles * a.heads + (int)std::min<long long>(wgs, kRowWorkers));
+        const bool sort = n_tiles * a.heads > 2 * cus;
+        if (a.head_dim == 64) launch_k(rswa_tile_kernel<64>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
+        else launch_k(rswa_tile_kernel<128>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
+        const hipError_t te = hipGetLastError();
+        return te == hipSuccess ? UOCR_HIP_OK : set_error(UOCR_HIP_EHIP, std::string("rswa launch: ") + hipGetErrorString(te));
     }
     const dim3 grid(rows, a.heads, a.n_chunks), block(kRswaWaves * 64);
     if (a.head_dim <= 64) launch_k(rswa_kernel<64>, grid, block, 0, st, a);
