@@ -344,12 +344,15 @@ int dense_experts_bm(const uocr_hip_moe_layer* L, int seq) {
                ? kDenseTiledBM
                : kDenseSkinnyBM;
 }
-// ... and of the unquantised shared MLP (every token: a plain GEMM)
+// ... and of the unquantised shared MLP (every token: a plain GEMM). Both
+// launches, us, 16-slot / 64-slot / 128-slot tiles at hidden 1280, width 1792: 64
+// tokens 20.8 / 22.2, 65 19.7 / 18.4, 127 26.4 / 18.4 / 29, 512 - / 19.8 / 29.2, 1024
+// - / 29.5 / 30.5, 2048 - / 57.2 / 48.7
 int dense_shared_bm(const uocr_hip_moe_layer* L, int seq) {
-    return (seq >= 128 && dense_shapes_ok(L->hidden, L->s_inter, true, kDenseTiledBM) &&
-            dense_shapes_ok(L->s_inter, L->hidden, false, kDenseTiledBM))
-               ? kDenseTiledBM
-               : kDenseSkinnyBM;
+    if (seq <= 64 || !dense_shapes_ok(L->hidden, L->s_inter, true, kDenseTiledBM) ||
+        !dense_shapes_ok(L->s_inter, L->hidden, false, kDenseTiledBM))
+        return kDenseSkinnyBM;
+    return seq <= 1024 ? kDenseTiledSmallBM : kDenseTiledBM;
 }
 // the layer runs the grouping kernels (prefill path, or unquantised experts)
 bool uses_grouping(const uocr_hip_moe_layer* L, int seq) { return L->experts_dense || use_prefill(L, seq); }

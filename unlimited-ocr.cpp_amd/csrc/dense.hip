@@ -18,32 +18,16 @@
 //     fragments straight from global memory into MFMA operand order), so the
 //     weight stream is limited by HBM, not by latency; the waves' partial sums
 //     meet in LDS.
-//   * dense_tiled_kernel -- 128 slots per tile (prefill). Activations are
-//     staged in LDS per 128-column k-tile, one k-tile ahead (double-buffered);
-//     each wave loads its own weight rows for the k-tile into registers and
-//     runs v_mfma_f32_32x32x16_f16 against the 4 staged 32-slot subtiles. Two
-//     workgroups per CU hide each other's load latency (measured faster than
-//     one workgroup per CU with the weights double-buffered in registers, and
-//     than 192-slot tiles).
+//   * dense_tile_kernel -- 64 or 128 slots per tile (prefill): both operands by
+//     DMA through LDS, several k-tiles ahead.
 // Gate/up (GU) pairs a gate block with the same up rows and writes
 // silu(g) * u as f16 act; down writes y (f16 per slot for the combine of the
 // grouped path, f32 per token for the shared MLP).
-#include "launch.hpp"
-
-#include <utility>
+#include "experts_prefill.hpp"
 
 namespace uocr_hip {
 
 namespace {
-
-template <typename F, int... I>
-__device__ __forceinline__ void sfor_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void sfor(F&& f) {
-    sfor_impl(f, std::make_integer_sequence<int, N>{});
-}
 
 // 8 consecutive activations as f16: f16 rows (AK 0) or bf16 rows (AK 1,
 // converted exactly within f16's range)
@@ -64,10 +48,6 @@ __device__ __forceinline__ f16x8 load_a8(const void* base, size_t idx) {
 }
 
 __device__ __forceinline__ f16x8 load_w8(const f16* p) { return *reinterpret_cast<const f16x8*>(p); }
-
-__device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
 
 struct TileDesc {
     int e, m0, rows, slot0;
@@ -168,121 +148,134 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Prefill-sized tiles (128 slots), two workgroups per CU. Workgroup = (tile,
-// output columns: GU 128 act columns = 4 waves x (32 gate + 32 up rows); down
-// 256 = 4 waves x 64 rows). Activations: wave w stages 32-slot subtile w of each 128-column
-// k-tile into LDS in 32x32x16 operand order (fragment (msub, s) = 1 KiB,
-// lane l: slot l % 32, columns s * 16 + 8 * (l / 32) .. + 8).
+// Prefill-sized tiles: BM (64 or 128) slots x 64 output columns (GU: the 64
+// gate and the 64 up rows of as many act columns) per workgroup of 2 x 2
+// waves, v_mfma_f32_32x32x16_f16 with the weights as the A operand (a lane
+// ends with 4 consecutive output columns of one slot).
+//   * A (gathered) and B rows come by 16-byte DMA in k-tiles of 64 columns,
+//     kStages - 1 k-tiles ahead, one barrier per k-tile; 8 lanes read a row's 128
+//     contiguous bytes (the operand-order DMA of the older kernel touched 32
+//     lines per instruction and had one k-tile in flight);
+//   * unit u (16 bytes) of row r sits at u ^ (r / 2 % 8): the operand reads of 16
+//     rows then cover all 64 banks;
+//   * the LDS reads are asm with counted waits (the compiler would wait for
+//     every DMA in flight before each of them).
+// Small batches are bound by latency (few workgroups, K / 64 dependent steps),
+// large ones by L2 and LDS reads. Measured against the older kernel (128 slots, one
+// k-tile of operand-order DMA ahead, 42 and 15 workgroups at 283 tokens), both
+// launches of the shared MLP: 283 tokens 97 -> 19.4 us, 1024 99 -> 29.5, 4096
+// 141 -> 100.
 // ---------------------------------------------------------------------------
-template <bool GU>
-__global__ __launch_bounds__(256, 2) void dense_tiled_kernel(DenseArgs a) {
-    constexpr int NS = 8;  // k16-steps per 128-column k-tile
-    constexpr int WB = 2;  // 32-row weight blocks per wave
-    __shared__ __attribute__((aligned(16))) f16 As[2][4 * NS * 512];
-    const int cols_wg = GU ? 128 : 256;
-    const int n_nt = a.n_out / cols_wg;
-    // XCD-aware order: the grid is a multiple of 8 and block b runs on XCD
-    // b % 8, so XCD x gets a contiguous run of (n-tile, tile) items: the tiles
-    // of one n-tile share its weight rows in that XCD's L2
-    const int per_xcd = gridDim.x / 8;
+template <int BM, bool GU>
+struct DenseTile {
+    static constexpr int BN = GU ? 128 : 64;  // weight rows
+    static constexpr int stage = (BM + BN) * 128;
+    static constexpr int fit = 81920 / stage;  // two workgroups per CU
+    static constexpr int stages = fit > 4 ? 4 : fit;
+    static constexpr int dmas = (BM + BN) / 32;  // per wave and k-tile
+};
+
+template <int BM, bool GU>
+__global__ __launch_bounds__(256, 2) void dense_tile_kernel(DenseArgs a, int n_tiles) {
+    using T = DenseTile<BM, GU>;
+    constexpr int JM = BM / 64, JN = GU ? 2 : 1;  // 32-slot and 32-weight-row blocks per wave
+    constexpr int kStages = T::stages, ND = T::dmas;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[kStages * T::stage];
+    const int n_nt = a.n_out / 64;
+    // XCD-aware order: block b runs on XCD b % 8; an XCD gets a contiguous run
+    // of (n-tile, tile) items, so the tiles of one n-tile share its weights in
+    // that XCD's L2
+    const int per_xcd = (n_nt * n_tiles + 7) / 8;
     const int item = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    const int n_tiles_grid = gridDim.x / n_nt;  // unused tail items exit below
-    (void)n_tiles_grid;
-    const int nt = item / (gridDim.x / n_nt), tile = item % (gridDim.x / n_nt);
-    if (nt >= n_nt) return;
+    if ((int)blockIdx.x / 8 >= per_xcd || item >= n_nt * n_tiles) return;
+    const int nt = item / n_tiles;
     TileDesc t;
-    if (!tile_desc(a, tile, kDenseTiledBM, t)) return;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int K = a.k, KT = K / kTileK;
+    if (!tile_desc(a, item % n_tiles, BM, t)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int K = a.k, KT = K / 64;
     const int l32 = lane & 31, lh = lane >> 5;
-    // A: this wave's 32-slot subtile
-    const int am = wave * 32 + l32;
-    const int slot = t.slot0 + min(am, t.rows - 1);
-    const int arow = a.slot_tok ? a.slot_tok[slot] : slot;
-    const f16* asrc = static_cast<const f16*>(a.a) + (size_t)arow * K + 8 * lh;
-    // B: this wave's weight rows
-    const f16* bsrc[WB];
+
+    // this wave's DMAs: 8 rows each (A rows, then weight rows)
+    const f16* src[ND];
 #pragma unroll
-    for (int b = 0; b < WB; ++b) {
-        const int row = GU ? (nt * 128 + wave * 32 + l32) : (nt * 256 + wave * 64 + b * 32 + l32);
-        const f16* w = (GU && b == 1) ? a.w1 : a.w0;
-        bsrc[b] = w + (size_t)t.e * a.w_stride + (size_t)row * K + 8 * lh;
-    }
-    f32x16 acc[WB][4];
-#pragma unroll
-    for (int b = 0; b < WB; ++b)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[b][i][r] = 0.f;
-    f16x8 ar[NS];
-    f16x8 bq[WB][NS];
-    auto load_a = [&](int kt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) ar[s] = *reinterpret_cast<const f16x8*>(asrc + kt * kTileK + s * 16);
-    };
-    auto write_a = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) *reinterpret_cast<f16x8*>(&As[buf][((wave * NS + s) * 64 + lane) * 8]) = ar[s];
-    };
-    auto load_b = [&](int kt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int b = 0; b < WB; ++b)
-#pragma unroll
-            for (int s = 0; s < NS; ++s) bq[b][s] = load_w8(bsrc[b] + kt * kTileK + s * 16);
-    };
-    auto compute = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            f16x8 af[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) af[i] = *reinterpret_cast<const f16x8*>(&As[buf][((i * NS + s) * 64 + lane) * 8]);
-#pragma unroll
-            for (int b = 0; b < WB; ++b)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[b][i] = mfma32(bq[b][s], af[i], acc[b][i]);
+    for (int d = 0; d < ND; ++d) {
+        const int r = (wave + 4 * d) * 8 + (lane >> 3), u = (lane & 7) ^ ((r >> 1) & 7);
+        const f16* row;
+        if (r < BM) {
+            const int slot = t.slot0 + min(r, t.rows - 1);
+            row = static_cast<const f16*>(a.a) + (size_t)(a.slot_tok ? a.slot_tok[slot] : slot) * K;
+        } else {
+            const int n = r - BM;
+            row = (GU && n >= 64 ? a.w1 : a.w0) + (size_t)t.e * a.w_stride + (size_t)(nt * 64 + (n & 63)) * K;
         }
-    };
-    // the weights of k-tile kt are issued at the top of its own iteration (no
-    // register double buffer: two workgroups per CU hide each other's
-    // latency), the activations one k-tile ahead through LDS
-    load_a(0);
-    write_a(0);
-    __syncthreads();
-    for (int kt = 0; kt < KT; ++kt) {
-        const bool more = kt + 1 < KT;
-        load_b(kt);
-        if (more) load_a(kt + 1);
-        compute(kt & 1);
-        if (more) write_a((kt + 1) & 1);
-        __syncthreads();
+        src[d] = row + u * 8;
     }
-    // D lane l: weight row 8 * (r / 4) + 4 * (l / 32) + r % 4 of the block, slot l % 32 of subtile i
+    auto issue = [&](int kt) {
+        uint8_t* dst = smem + (kt % kStages) * T::stage;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int mm = i * 32 + l32;
+        for (int d = 0; d < ND; ++d) load_lds16(src[d] + kt * 64, dst + (wave + 4 * d) * 1024);
+    };
+    // operand reads of k-step s: row l32 of a 32-row block, unit 2 s + lh
+    uint32_t off[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) off[s] = l32 * 128 + (((2 * s + lh) ^ ((l32 >> 1) & 7)) << 4);
+
+    f32x16 acc[JN][JM];
+#pragma unroll
+    for (int n = 0; n < JN; ++n)
+#pragma unroll
+        for (int m = 0; m < JM; ++m) acc[n][m] = f32x16{};
+    const uint32_t base = lds_addr(smem);
+    for (int kt = 0; kt < kStages - 1 && kt < KT; ++kt) issue(kt);
+    for (int kt = 0; kt < KT; ++kt) {
+        // this wave's part of k-tile kt has landed; after the barrier every
+        // wave's has, and k-tile kt - 1 is read
+        if (kt + kStages - 2 < KT) vm_wait<ND * (kStages - 2)>();
+        else vm_wait<0>();
+        asm volatile("s_barrier" ::: "memory");
+        if (kt + kStages - 1 < KT) issue(kt + kStages - 1);
+        const uint32_t st = base + (kt % kStages) * T::stage;
+        const uint32_t sa = st + wm * (32 * JM) * 128, sb = st + (BM + wn * 32) * 128;
+        f16x8 af[2][JM], bf[2][JN];
+        auto read = [&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            static_for<JM>([&](auto m) { lds_read16<decltype(m)::value * 4096>(af[s & 1][decltype(m)::value], sa + off[s]); });
+            static_for<JN>([&](auto n) { lds_read16<decltype(n)::value * 8192>(bf[s & 1][decltype(n)::value], sb + off[s]); });
+        };
+        read(std::integral_constant<int, 0>{});
+        static_for<4>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            if constexpr (s < 3) read(std::integral_constant<int, s + 1>{});
+            lgkm_wait<(s < 3 ? JM + JN : 0)>();
+#pragma unroll
+            for (int m = 0; m < JM; ++m) tie(af[s & 1][m]);
+#pragma unroll
+            for (int n = 0; n < JN; ++n) tie(bf[s & 1][n]);
+#pragma unroll
+            for (int n = 0; n < JN; ++n)
+#pragma unroll
+                for (int m = 0; m < JM; ++m) acc[n][m] = mfma32(bf[s & 1][n], af[s & 1][m], acc[n][m]);
+        });
+    }
+    // D lane l: weight row 8 * (r / 4) + 4 * (l / 32) + r % 4 of the block, slot l % 32
+#pragma unroll
+    for (int m = 0; m < JM; ++m) {
+        const int mm = (wm * JM + m) * 32 + l32;
         if (mm >= t.rows) continue;
-        const size_t orow = (size_t)(t.slot0 + mm) * a.n_out;
+        const size_t orow = (size_t)(t.slot0 + mm) * a.n_out + nt * 64 + wn * 32;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int r0 = 8 * q + 4 * lh;
+            const size_t o = orow + 8 * q + 4 * lh;
+            const f32x16& v = acc[0][m];
             if constexpr (GU) {
-                const size_t o = orow + nt * 128 + wave * 32 + r0;
-                store_f16x4(a.out16 + o, silu_mul_f(acc[0][i][4 * q], acc[1][i][4 * q]),
-                            silu_mul_f(acc[0][i][4 * q + 1], acc[1][i][4 * q + 1]),
-                            silu_mul_f(acc[0][i][4 * q + 2], acc[1][i][4 * q + 2]),
-                            silu_mul_f(acc[0][i][4 * q + 3], acc[1][i][4 * q + 3]), a.status);
+                const f32x16& u = acc[JN - 1][m];
+                store_f16x4(a.out16 + o, silu_mul_f(v[4 * q], u[4 * q]), silu_mul_f(v[4 * q + 1], u[4 * q + 1]),
+                            silu_mul_f(v[4 * q + 2], u[4 * q + 2]), silu_mul_f(v[4 * q + 3], u[4 * q + 3]), a.status);
+            } else if (a.out32) {
+                *reinterpret_cast<f32x4*>(a.out32 + o) = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
             } else {
-#pragma unroll
-                for (int b = 0; b < WB; ++b) {
-                    const size_t o = orow + nt * 256 + wave * 64 + b * 32 + r0;
-                    if (a.out32)
-                        *reinterpret_cast<f32x4*>(a.out32 + o) =
-                            f32x4{acc[b][i][4 * q], acc[b][i][4 * q + 1], acc[b][i][4 * q + 2], acc[b][i][4 * q + 3]};
-                    else
-                        store_f16x4(a.out16 + o, acc[b][i][4 * q], acc[b][i][4 * q + 1], acc[b][i][4 * q + 2],
-                                    acc[b][i][4 * q + 3], a.status);
-                }
+                store_f16x4(a.out16 + o, v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], a.status);
             }
         }
     }
@@ -294,7 +287,7 @@ __global__ __launch_bounds__(256, 2) void dense_tiled_kernel(DenseArgs a) {
 bool dense_shapes_ok(int k, int n_out, bool gate_up, int bm) {
     if (k <= 0 || n_out <= 0 || k % kTileK) return false;
     if (bm == kDenseSkinnyBM) return n_out % 16 == 0 && (k / 32) % 4 == 0;
-    if (bm == kDenseTiledBM) return n_out % (gate_up ? 128 : 256) == 0;
+    if (bm == kDenseTiledBM || bm == kDenseTiledSmallBM) return n_out % 64 == 0;
     return false;
 }
 
@@ -375,15 +368,14 @@ hipError_t launch_dense(const DenseArgs& a, bool gate_up, int bm, int max_tiles,
         return gate_up ? launch_skinny<true, 0>(a, n_tiles, st) : launch_skinny<false, 0>(a, n_tiles, st);
     }
     if (a.a_kind != 0) return hipErrorInvalidValue;
-    const int n_nt = a.n_out / (gate_up ? 128 : 256);
-    const int blocks = (n_tiles * n_nt + 7) / 8 * 8;
-    // the in-kernel item map needs blocks to be a multiple of n_nt as well
-    int grid = blocks;
-    while (grid % n_nt) grid += 8;
-    if (gate_up)
-        launch_k(dense_tiled_kernel<true>, dim3(grid), dim3(256), 0, st, a);
-    else
-        launch_k(dense_tiled_kernel<false>, dim3(grid), dim3(256), 0, st, a);
+    const int grid = (n_tiles * (a.n_out / 64) + 7) / 8 * 8;
+    if (bm == 64) {
+        if (gate_up) launch_k((dense_tile_kernel<64, true>), dim3(grid), dim3(256), 0, st, a, n_tiles);
+        else launch_k((dense_tile_kernel<64, false>), dim3(grid), dim3(256), 0, st, a, n_tiles);
+    } else {
+        if (gate_up) launch_k((dense_tile_kernel<128, true>), dim3(grid), dim3(256), 0, st, a, n_tiles);
+        else launch_k((dense_tile_kernel<128, false>), dim3(grid), dim3(256), 0, st, a, n_tiles);
+    }
     return hipGetLastError();
 }
 

@@ -217,6 +217,7 @@ hipError_t launch_combine(const CombineArgs& c, hipStream_t st);
 // [experts][rows][cols] on the device (dense.hip).
 constexpr int kDenseSkinnyBM = 16;   // decode-sized tiles
 constexpr int kDenseTiledBM = 128;   // prefill-sized tiles
+constexpr int kDenseTiledSmallBM = 64;  // and the smaller ones of a short prefill (shared MLP)
 struct DenseArgs {
     const void* a;          // A rows: f16 (x16 / act) or bf16 (the layer input x)
     int a_kind;             // 0 f16, 1 bf16
