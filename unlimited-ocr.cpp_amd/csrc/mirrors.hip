@@ -84,99 +84,116 @@ __global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-        for (int k0 = 0; k0 < K; k0 += kMKC) {
-            const int kc = min(kMKC, K - k0);  // a multiple of 32
-            // activations: 64 rows x 16 runs of 8 columns
+        // The next chunk's loads are issued into registers before the current
+        // chunk's MFMAs and written to LDS after them: a chunk then costs its
+        // MFMAs and LDS traffic, not a round trip to memory. Rows past the
+        // last and columns past K load a valid address and are stored as 0.
+        const float* arow[4];
+        bool alive[4];
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {  // 64 rows x 16 runs of 8 columns
+            const int slot = m0 + ((tid + 256 * it) >> 4);
+            alive[it] = slot < rows;
+            const int sl = alive[it] ? slot : m0;
+            long long row;
+            if constexpr (MODE == kGateUp) row = a.assign_token[(size_t)e * a.cap + sl];
+            else if constexpr (MODE == kDown) row = (long long)e * a.cap + sl;
+            else row = sl;
+            arow[it] = a.a + (size_t)row * K;
+        }
+        const int c8 = tid & 15;
+        constexpr int NW4 = WFMT == 0 ? NM : 4 * NM;  // 16-byte weight loads per thread
+        f32x4 ar[4][2];
+        u32x4 wr[NW4];
+        float sr[NM], zr[NM];  // INT4: a 32-column run lies in one group (group % 32 == 0)
+        auto load = [&](int k0) {
+            const int ka = min(k0 + c8 * 8, K - 8);
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
-                const int u = tid + 256 * it, m = u >> 4, c8 = u & 15;
-                f16x8 v;
-                const int slot = m0 + m;
-                if (slot < rows && c8 * 8 < kc) {
-                    long long row;
-                    if constexpr (MODE == kGateUp) row = a.assign_token[(size_t)e * a.cap + slot];
-                    else if constexpr (MODE == kDown) row = (long long)e * a.cap + slot;
-                    else row = slot;
-                    const float* src = a.a + (size_t)row * K + k0 + c8 * 8;
-                    const f32x4 p = *reinterpret_cast<const f32x4*>(src);
-                    const f32x4 q = *reinterpret_cast<const f32x4*>(src + 4);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        v[i] = (f16)p[i];
-                        v[4 + i] = (f16)q[i];
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) v[i] = (f16)0.0f;
-                }
-                // fragment (m / 16, k-step c8 / 4), lane (m % 16) + 16 * (c8 % 4)
-                const int frag = (m >> 4) * 4 + (c8 >> 2);
-                *reinterpret_cast<f16x8*>(As + (size_t)frag * kMFrag + ((m & 15) + 16 * (c8 & 3)) * 8) = v;
+                ar[it][0] = *reinterpret_cast<const f32x4*>(arow[it] + ka);
+                ar[it][1] = *reinterpret_cast<const f32x4*>(arow[it] + ka + 4);
             }
-            // weights
             if constexpr (WFMT == 0) {
                 // NM x 64 rows x 4 runs of 32 columns (16 packed bytes)
+                const int n = tid >> 2, kk = min(k0 + (tid & 3) * 32, K - 32);
 #pragma unroll
                 for (int it = 0; it < NM; ++it) {
-                    const int u = tid + 256 * it, mat = u >> 8, n = (u >> 2) & 63, c32 = u & 3;
-                    const uint8_t* P = mat ? a.p1 : a.p0;
-                    const float* S = mat ? a.s1 : a.s0;
-                    const float* Z = mat ? a.z1 : a.z0;
-                    const long long ps = mat ? a.pstride1 : a.pstride0, ss = mat ? a.sstride1 : a.sstride0;
-                    const int ng = mat ? a.ng1 : a.ng0;
-                    const int kk = k0 + c32 * 32;
-                    f16x8 v[4];
-                    if (c32 * 32 < kc) {
-                        const uint8_t* prow = P + (size_t)e * ps + (size_t)(n0 + n) * packed_row + kk / 2;
-                        u32x4 w;
-                        __builtin_memcpy(&w, prow, 16);  // 16-byte aligned when K % 32 == 0
-                        const size_t sidx = (size_t)e * ss + (size_t)(n0 + n) * ng;
-#pragma unroll
-                        for (int r8 = 0; r8 < 4; ++r8) {
-                            const int g = (kk + r8 * 8) / a.group;
-                            const float sc = S[sidx + g], zr = Z[sidx + g];
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) {
-                                const uint32_t byte = (w[(r8 * 8 + i) >> 3] >> (8 * (((r8 * 8 + i) & 7) >> 1))) & 0xffu;
-                                const uint32_t q = (i & 1) ? (byte >> 4) : (byte & 0x0fu);
-                                v[r8][i] = (f16)(((float)q - zr) * sc);
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int r8 = 0; r8 < 4; ++r8)
-#pragma unroll
-                            for (int i = 0; i < 8; ++i) v[r8][i] = (f16)0.0f;
-                    }
-                    // run r8 of k-step c32 -> lane (n % 16) + 16 * r8
-#pragma unroll
-                    for (int r8 = 0; r8 < 4; ++r8) {
-                        const int frag = (mat * 4 + (n >> 4)) * 4 + c32;
-                        *reinterpret_cast<f16x8*>(Bs + (size_t)frag * kMFrag + ((n & 15) + 16 * r8) * 8) = v[r8];
-                    }
+                    const uint8_t* prow = (it ? a.p1 : a.p0) + (size_t)e * (it ? a.pstride1 : a.pstride0) +
+                                          (size_t)(n0 + n) * packed_row + kk / 2;
+                    __builtin_memcpy(&wr[it], prow, 16);  // 16-byte aligned when K % 32 == 0
+                    const size_t sidx = (size_t)e * (it ? a.sstride1 : a.sstride0) +
+                                        (size_t)(n0 + n) * (it ? a.ng1 : a.ng0) + kk / a.group;
+                    sr[it] = (it ? a.s1 : a.s0)[sidx];
+                    zr[it] = (it ? a.z1 : a.z0)[sidx];
                 }
             } else {
                 // NM x 64 rows x 16 runs of 8 bf16
 #pragma unroll
                 for (int it = 0; it < 4 * NM; ++it) {
-                    const int u = tid + 256 * it, mat = u >> 10, n = (u >> 4) & 63, c8 = u & 15;
-                    u32x4 w = {0u, 0u, 0u, 0u};
-                    if (c8 * 8 < kc) {
-                        const uint16_t* wm = MODE == kPlain ? a.wplain : (mat ? a.w1 : a.w0)[e];
-                        const uint16_t* row = wm + (size_t)(n0 + n) * K + k0 + c8 * 8;
-                        w = *reinterpret_cast<const u32x4*>(row);
+                    const int mat = it >> 2, n = ((tid + 256 * it) >> 4) & 63;
+                    const uint16_t* wm = MODE == kPlain ? a.wplain : (mat ? a.w1 : a.w0)[e];
+                    wr[it] = *reinterpret_cast<const u32x4*>(wm + (size_t)(n0 + n) * K + ka);
+                }
+            }
+        };
+        auto store = [&](int kc) {
+#pragma unroll
+            for (int it = 0; it < 4; ++it) {
+                const int m = (tid + 256 * it) >> 4;
+                const bool on = alive[it] && c8 * 8 < kc;
+                f16x8 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = on ? (f16)ar[it][0][i] : (f16)0.0f;
+                    v[4 + i] = on ? (f16)ar[it][1][i] : (f16)0.0f;
+                }
+                // fragment (m / 16, k-step c8 / 4), lane (m % 16) + 16 * (c8 % 4)
+                const int frag = (m >> 4) * 4 + (c8 >> 2);
+                *reinterpret_cast<f16x8*>(As + (size_t)frag * kMFrag + ((m & 15) + 16 * (c8 & 3)) * 8) = v;
+            }
+            if constexpr (WFMT == 0) {
+                const int n = tid >> 2, c32 = tid & 3;
+                const bool on = c32 * 32 < kc;
+#pragma unroll
+                for (int it = 0; it < NM; ++it) {
+                    const u32x4 w = wr[it];
+                    // run r8 of k-step c32 -> lane (n % 16) + 16 * r8
+#pragma unroll
+                    for (int r8 = 0; r8 < 4; ++r8) {
+                        f16x8 v;
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            const float q = (float)((w[r8] >> (4 * i)) & 0xfu);
+                            v[i] = on ? (f16)((q - zr[it]) * sr[it]) : (f16)0.0f;
+                        }
+                        const int frag = (it * 4 + (n >> 4)) * 4 + c32;
+                        *reinterpret_cast<f16x8*>(Bs + (size_t)frag * kMFrag + ((n & 15) + 16 * r8) * 8) = v;
                     }
+                }
+            } else {
+                const bool on = c8 * 8 < kc;
+#pragma unroll
+                for (int it = 0; it < 4 * NM; ++it) {
+                    const int mat = it >> 2, n = ((tid + 256 * it) >> 4) & 63;
+                    const u32x4 w = wr[it];
                     f16x8 v;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        v[2 * i] = (f16)bf16_bits_to_f32(w[i] & 0xffffu);
-                        v[2 * i + 1] = (f16)__uint_as_float(w[i] & 0xffff0000u);
+                        v[2 * i] = on ? (f16)bf16_bits_to_f32(w[i] & 0xffffu) : (f16)0.0f;
+                        v[2 * i + 1] = on ? (f16)__uint_as_float(w[i] & 0xffff0000u) : (f16)0.0f;
                     }
                     const int frag = (mat * 4 + (n >> 4)) * 4 + (c8 >> 2);
                     *reinterpret_cast<f16x8*>(Bs + (size_t)frag * kMFrag + ((n & 15) + 16 * (c8 & 3)) * 8) = v;
                 }
             }
+        };
+        load(0);
+        for (int k0 = 0; k0 < K; k0 += kMKC) {
+            const int kc = min(kMKC, K - k0);  // a multiple of 32
+            store(kc);
             __syncthreads();
+            if (k0 + kMKC < K) load(k0 + kMKC);
+            __builtin_amdgcn_sched_barrier(0);  // (issued here, not sunk to their use)
             // wave w: n-subtile w of every matrix, all four m-subtiles
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
