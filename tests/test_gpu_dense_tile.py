@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("seq,hidden,inter,n_shared", [
     (65, 1280, 128, 2), (128, 256, 896, 2), (129, 1280, 128, 14), (1023, 128, 128, 1), (1024, 384, 128, 3),
-    (1025, 384, 128, 3), (1300, 1280, 128, 1),
+    (1025, 384, 128, 3), (1300, 1280, 128, 1), (3300, 1280, 128, 1),
 ])
 def test_shared_mlp_tiles(dev, seq, hidden, inter, n_shared):
     from uocr_hip import synth
@@ -22,7 +22,7 @@ def test_shared_mlp_tiles(dev, seq, hidden, inter, n_shared):
     check_parity(L, x, dev, sample=24, label=f"shared H={hidden} I={inter} S={n_shared}")
 
 
-@pytest.mark.parametrize("seq,hidden,inter", [(256, 384, 128), (400, 128, 384), (700, 640, 256)])
+@pytest.mark.parametrize("seq,hidden,inter", [(256, 384, 128), (400, 128, 384), (700, 640, 256), (1111, 1280, 896)])
 def test_routed_expert_tiles(dev, seq, hidden, inter):
     from uocr_hip import synth
     L = synth.random_layer_bf16(seed=seq, hidden=hidden, inter=inter, n_experts=6, top_k=3, n_shared=1)

@@ -334,15 +334,24 @@ bool use_stream(const uocr_hip_moe_layer* L, int seq, int x_dtype) {
 
 
 // Tile rows of the unquantised expert kernels: decode-sized tiles below the
-// prefill threshold, 128-slot MFMA tiles from there (when the shapes allow)
+// prefill threshold, from there (when the shapes allow) 64 or 128 slots. 64 up to
+// 56 rows per expert on average, where most experts fill one such tile: gate/up +
+// down, us, 64 / 128 slots at 64 experts, top-6: 256 tokens 106 / 116, 512 119 /
+// 131, 768 172 / 143, 1111 170 / 154, 2048 258 / 236.
 int dense_experts_bm(const uocr_hip_moe_layer* L, int seq) {
-    if (seq < kPrefillMinSeq) return kDenseSkinnyBM;
-    // the large-tile kernel with f16 weight fragments DMA'd to LDS (K in {896, 1280})
-    if (prefill_big_ok(L->hidden, L->inter)) return kPrefillBigTileRows;
-    return (dense_shapes_ok(L->hidden, L->inter, true, kDenseTiledBM) &&
-            dense_shapes_ok(L->inter, L->hidden, false, kDenseTiledBM))
-               ? kDenseTiledBM
-               : kDenseSkinnyBM;
+    if (seq < kPrefillMinSeq || !dense_shapes_ok(L->hidden, L->inter, true, kDenseTiledBM) ||
+        !dense_shapes_ok(L->inter, L->hidden, false, kDenseTiledBM))
+        return kDenseSkinnyBM;
+    return (long long)seq * L->top_k <= 56ll * L->n_experts ? kDenseTiledSmallBM : kDenseTiledBM;
+}
+// ... and of the INT4 expert kernels. 64 slots, two workgroups per CU, up to 56
+// rows per expert on average; above, 256 slots (experts of at most 128 rows in half
+// mode) for the shapes it is built for, else 128. Gate/up + down, us, 64 / 128 / 256 slots
+// at 64 experts, top-6, group 32: 256 tokens 75 / 91 / 101, 512 83 / 99 / 102, 768 120 /
+// 105 / 108, 1024 131 / 114 / 108, 2048 219 / 193 / 189, 4096 402 / 329 / 299.
+int int4_bm(const uocr_hip_moe_layer* L, int seq) {
+    if ((long long)seq * L->top_k <= 56ll * L->n_experts) return kPrefillSmallTileRows;
+    return prefill_big_ok(L->hidden, L->inter) ? kPrefillBigTileRows : kPrefillTileRows;
 }
 // ... and of the unquantised shared MLP (every token: a plain GEMM). Both
 // launches, us, 16-slot / 64-slot / 128-slot tiles at hidden 1280, width 1792: 64
@@ -364,7 +373,7 @@ WsPlan plan(const uocr_hip_moe_layer* L, int seq) {
     p.bm = L->experts_dense ? dense_experts_bm(L, seq)
            : !use_prefill(L, seq)
                ? kDecodeTileRows
-               : (prefill_big_ok(L->hidden, L->inter) ? kPrefillBigTileRows : kPrefillTileRows);
+               : int4_bm(L, seq);
     p.max_tiles = (seq * L->top_k) / p.bm + L->n_experts + L->n_virtual * ((seq + p.bm - 1) / p.bm) + 1;
     size_t o = 0;
     auto take = [&](size_t bytes) {
@@ -1037,38 +1046,7 @@ int uocr_hip_moe_layer_forward(const uocr_hip_moe_layer* L, const void* x, int x
     HIP_TRY(launch_group(g, st), "group launch");
     stage(2);
     const f16* y16 = (const f16*)(ws + p.y);
-    if (L->experts_dense && p.bm == kPrefillBigTileRows) {
-        ExpertArgs gu{};
-        gu.a = x16;
-        gu.gather = 1;
-        gu.w0 = reinterpret_cast<const uint8_t*>(L->egate);
-        gu.w1 = reinterpret_cast<const uint8_t*>(L->eup);
-        gu.w_stride = (long long)L->inter * L->hidden * 2;
-        gu.n_rows = L->inter;
-        gu.k = L->hidden;
-        gu.bm = p.bm;
-        gu.slot_tok = g.slot_tok;
-        gu.counts = g.counts;
-        gu.offsets = g.offsets;
-        gu.tile_e = g.tile_e;
-        gu.tile_m0 = g.tile_m0;
-        gu.tile_info = g.tile_info;
-        gu.n_tiles = g.n_tiles;
-        gu.act_out = (f16*)(ws + p.act);
-        gu.status = &L->sync->error;
-        HIP_TRY(launch_experts_prefill_dense(gu, true, p.max_tiles, st), "gate/up launch");
-        stage(3);
-        ExpertArgs dn = gu;
-        dn.a = gu.act_out;
-        dn.gather = 0;
-        dn.w0 = reinterpret_cast<const uint8_t*>(L->edown);
-        dn.w1 = nullptr;
-        dn.n_rows = L->hidden;
-        dn.k = L->inter;
-        dn.act_out = nullptr;
-        dn.y_out = (f16*)(ws + p.y);
-        HIP_TRY(launch_experts_prefill_dense(dn, false, p.max_tiles, st), "down launch");
-    } else if (L->experts_dense) {
+    if (L->experts_dense) {
         DenseArgs gu{};
         gu.a = x16;
         gu.a_kind = 0;

@@ -148,9 +148,9 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Prefill-sized tiles: BM (64 or 128) slots x 64 output columns (GU: the 64
-// gate and the 64 up rows of as many act columns) per workgroup of 2 x 2
-// waves, v_mfma_f32_32x32x16_f16 with the weights as the A operand (a lane
+// Prefill-sized tiles: BM (64 or 128) slots x NJ 64-row blocks of weights (GU:
+// the gate and the up rows of 64 act columns; down: 64 or 128 output columns) per
+// workgroup of 2 x 2 waves, v_mfma_f32_32x32x16_f16 with the weights as the A operand (a lane
 // ends with 4 consecutive output columns of one slot).
 //   * A (gathered) and B rows come by 16-byte DMA in k-tiles of 64 columns,
 //     kStages - 1 k-tiles ahead, one barrier per k-tile; 8 lanes read a row's 128
@@ -166,22 +166,24 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseArgs a) {
 // launches of the shared MLP: 283 tokens 97 -> 19.4 us, 1024 99 -> 29.5, 4096
 // 141 -> 100.
 // ---------------------------------------------------------------------------
-template <int BM, bool GU>
+template <int BM, int NJ>
 struct DenseTile {
-    static constexpr int BN = GU ? 128 : 64;  // weight rows
+    static constexpr int BN = 64 * NJ;  // weight rows
     static constexpr int stage = (BM + BN) * 128;
     static constexpr int fit = 81920 / stage;  // two workgroups per CU
     static constexpr int stages = fit > 4 ? 4 : fit;
     static constexpr int dmas = (BM + BN) / 32;  // per wave and k-tile
 };
 
-template <int BM, bool GU>
+template <int BM, bool GU, int NJ>
 __global__ __launch_bounds__(256, 2) void dense_tile_kernel(DenseArgs a, int n_tiles) {
-    using T = DenseTile<BM, GU>;
-    constexpr int JM = BM / 64, JN = GU ? 2 : 1;  // 32-slot and 32-weight-row blocks per wave
+    static_assert(!GU || NJ == 2, "one gate and one up block");
+    using T = DenseTile<BM, NJ>;
+    constexpr int JM = BM / 64, JN = NJ;      // 32-slot and 32-weight-row blocks per wave
+    constexpr int NC = GU ? 64 : 64 * NJ;     // output columns
     constexpr int kStages = T::stages, ND = T::dmas;
     __shared__ __attribute__((aligned(16))) uint8_t smem[kStages * T::stage];
-    const int n_nt = a.n_out / 64;
+    const int n_nt = a.n_out / NC;
     // XCD-aware order: block b runs on XCD b % 8; an XCD gets a contiguous run
     // of (n-tile, tile) items, so the tiles of one n-tile share its weights in
     // that XCD's L2
@@ -207,7 +209,7 @@ __global__ __launch_bounds__(256, 2) void dense_tile_kernel(DenseArgs a, int n_t
             row = static_cast<const f16*>(a.a) + (size_t)(a.slot_tok ? a.slot_tok[slot] : slot) * K;
         } else {
             const int n = r - BM;
-            row = (GU && n >= 64 ? a.w1 : a.w0) + (size_t)t.e * a.w_stride + (size_t)(nt * 64 + (n & 63)) * K;
+            row = (GU && n >= 64 ? a.w1 : a.w0) + (size_t)t.e * a.w_stride + (size_t)(nt * NC + (GU ? n & 63 : n)) * K;
         }
         src[d] = row + u * 8;
     }
@@ -263,21 +265,23 @@ __global__ __launch_bounds__(256, 2) void dense_tile_kernel(DenseArgs a, int n_t
     for (int m = 0; m < JM; ++m) {
         const int mm = (wm * JM + m) * 32 + l32;
         if (mm >= t.rows) continue;
-        const size_t orow = (size_t)(t.slot0 + mm) * a.n_out + nt * 64 + wn * 32;
+        const size_t orow = (size_t)(t.slot0 + mm) * a.n_out + nt * NC + wn * 32;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const size_t o = orow + 8 * q + 4 * lh;
-            const f32x16& v = acc[0][m];
-            if constexpr (GU) {
-                const f32x16& u = acc[JN - 1][m];
-                store_f16x4(a.out16 + o, silu_mul_f(v[4 * q], u[4 * q]), silu_mul_f(v[4 * q + 1], u[4 * q + 1]),
-                            silu_mul_f(v[4 * q + 2], u[4 * q + 2]), silu_mul_f(v[4 * q + 3], u[4 * q + 3]), a.status);
-            } else if (a.out32) {
-                *reinterpret_cast<f32x4*>(a.out32 + o) = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
-            } else {
-                store_f16x4(a.out16 + o, v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], a.status);
+        for (int n = 0; n < (GU ? 1 : JN); ++n)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const size_t o = orow + n * 64 + 8 * q + 4 * lh;
+                const f32x16& v = acc[n][m];
+                if constexpr (GU) {
+                    const f32x16& u = acc[JN - 1][m];
+                    store_f16x4(a.out16 + o, silu_mul_f(v[4 * q], u[4 * q]), silu_mul_f(v[4 * q + 1], u[4 * q + 1]),
+                                silu_mul_f(v[4 * q + 2], u[4 * q + 2]), silu_mul_f(v[4 * q + 3], u[4 * q + 3]), a.status);
+                } else if (a.out32) {
+                    *reinterpret_cast<f32x4*>(a.out32 + o) = f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+                } else {
+                    store_f16x4(a.out16 + o, v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3], a.status);
+                }
             }
-        }
     }
 }
 
@@ -368,15 +372,17 @@ hipError_t launch_dense(const DenseArgs& a, bool gate_up, int bm, int max_tiles,
         return gate_up ? launch_skinny<true, 0>(a, n_tiles, st) : launch_skinny<false, 0>(a, n_tiles, st);
     }
     if (a.a_kind != 0) return hipErrorInvalidValue;
-    const int grid = (n_tiles * (a.n_out / 64) + 7) / 8 * 8;
-    if (bm == 64) {
-        if (gate_up) launch_k((dense_tile_kernel<64, true>), dim3(grid), dim3(256), 0, st, a, n_tiles);
-        else launch_k((dense_tile_kernel<64, false>), dim3(grid), dim3(256), 0, st, a, n_tiles);
-    } else {
-        if (gate_up) launch_k((dense_tile_kernel<128, true>), dim3(grid), dim3(256), 0, st, a, n_tiles);
-        else launch_k((dense_tile_kernel<128, false>), dim3(grid), dim3(256), 0, st, a, n_tiles);
-    }
-    return hipGetLastError();
+    auto launch = [&](auto kernel, int cols) {
+        launch_k(kernel, dim3((n_tiles * (a.n_out / cols) + 7) / 8 * 8), dim3(256), 0, st, a, n_tiles);
+        return hipGetLastError();
+    };
+    // down: 128 output columns per workgroup (twice the MFMAs per LDS read) once
+    // that leaves a workgroup per CU (grouped experts at 1111 tokens 73.8 -> 56.9
+    // us; the shared MLP at 1536 tokens would lose 7 us)
+    const bool wide = a.n_out % 128 == 0 && n_tiles * (a.n_out / 128) >= 256;
+    if (gate_up) return bm == 64 ? launch(dense_tile_kernel<64, true, 2>, 64) : launch(dense_tile_kernel<128, true, 2>, 64);
+    if (wide) return bm == 64 ? launch(dense_tile_kernel<64, false, 2>, 128) : launch(dense_tile_kernel<128, false, 2>, 128);
+    return bm == 64 ? launch(dense_tile_kernel<64, false, 1>, 64) : launch(dense_tile_kernel<128, false, 1>, 64);
 }
 
 }  // namespace uocr_hip

@@ -1,20 +1,10 @@
-// Prefill-sized grouped INT4 expert GEMM (MFMA-bound): dequantise the INT4
-// weights into LDS-staged f16 tiles feeding v_mfma_f32_16x16x32_f16.
-//
-// Counterpart of the reference's grouped pair moe_grouped_gate_up_int4 /
-// moe_grouped_down_int4 (src/kernels/cuda/moe_gemm_int4.cu:535-732), which
-// stages bf16 panels for mma.sync m16n8k16. Here:
-//   * work items are (m-tile of up to 128 grouped slots of one expert, n-tile)
-//     taken from the device tile list, so skewed experts (Zipf routing) simply
-//     own more m-tiles and every CU gets full 128-row tiles;
-//   * a workgroup (4 waves, 2 x 2) computes 128 slots x 128 weight rows; the
-//     fused gate/up pass pairs 64 gate rows with the same 64 up rows so SiLU(g)*u
-//     is formed in registers and written once as f16 `act`;
-//   * per 128-column k-tile, activation rows are copied global->LDS directly
-//     (gathered through the slot->token list) and the 8 KiB of packed weights
-//     are dequantised once per workgroup, exactly, into f16 fragments; both land
-//     in MFMA fragment order (1 KiB per 16x32 fragment, lane-contiguous), so every
-//     LDS read is a linear 1 KiB wave read.
+// Asm loads, LDS accesses and counted waits of the tiled expert kernels, and
+// the large-tile INT4 expert GEMM of a large prefill (MFMA-bound). Work items are
+// (m-tile of up to 256 grouped slots of one expert, n-tile) taken from the device
+// tile list, so skewed experts (Zipf routing) simply own more m-tiles; the fused
+// gate/up pass pairs gate rows with the same up rows so SiLU(g)*u is formed in
+// registers and written once as f16 `act`. experts_tile.hpp has the kernel of
+// smaller batches.
 #include <type_traits>
 #include <utility>
 
@@ -75,158 +65,11 @@ __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
-constexpr int kPreBM = 128;               // slots per m-tile (generic kernel)
-constexpr int kPreBN = 128;               // weight rows per workgroup
 constexpr int kBigBM = kPrefillBigTileRows; // slots per m-tile (large-tile kernel)
 constexpr int kFragHalfs = 64 * 8;        // f16 per 1 KiB fragment
 
-template <int GPT, bool GU, bool ZP>
-__global__ __launch_bounds__(256) void experts_prefill_kernel(ExpertArgs a) {
-    // A: 8 m-subtiles x 4 k-steps; B: 8 row blocks x 4 k-steps (fragments of 1 KiB)
-    __shared__ __attribute__((aligned(16))) f16 As[8 * 4 * kFragHalfs];
-    __shared__ __attribute__((aligned(16))) f16 Bs[8 * 4 * kFragHalfs];
-    const int n_ntiles = GU ? (a.n_rows / (kPreBN / 2)) : (a.n_rows / kPreBN);
-    const int tile = blockIdx.x / n_ntiles, ntile = blockIdx.x % n_ntiles;
-    const int n_tiles = *a.n_tiles;
-    const int e = a.tile_e[tile], m0 = a.tile_m0[tile];
-    if (tile >= n_tiles) return;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int rows = min(kPreBM, a.counts[e] - m0);
-    const int slot0 = a.offsets[e] + m0;
-    const int K = a.k, KT = K / kTileK;
-    const int NG = scale_row_stride(K, kTileK / GPT);
-
-    // this wave's A rows for the DMA: m-subtiles (wave + 4i), row lane % 16
-    const f16* arow[2];
-    bool alive[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int m = (wave + 4 * i) * 16 + (lane & 15);
-        alive[i] = m < rows;
-        const int slot = slot0 + (alive[i] ? m : 0);
-        const int row = a.gather ? a.slot_tok[slot] : slot;
-        arow[i] = a.a + (size_t)row * K + 8 * (lane >> 4);
-    }
-    // this thread's B row blocks for the dequant: rb = wave and rb = wave + 4
-    // (GU: 0..3 gate rows n0..n0+63, 4..7 the same up rows)
-    const uint8_t* bsrc[2];
-    const f16* ssrc[2];
-    const f16* zsrc[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int rbl = wave + 4 * i;
-        int grow;  // global weight row block
-        const uint8_t* wbase;
-        const uint16_t* sbase;
-        const uint16_t* zbase;
-        if constexpr (GU) {
-            grow = ntile * 4 + (rbl & 3);
-            wbase = (rbl < 4 ? a.w0 : a.w1) + (size_t)e * a.w_stride;
-            sbase = (rbl < 4 ? a.s0 : a.s1) + (size_t)e * a.s_stride;
-            zbase = (rbl < 4 ? a.z0 : a.z1) + (size_t)e * a.s_stride;
-        } else {
-            grow = ntile * 8 + rbl;
-            wbase = a.w0 + (size_t)e * a.w_stride;
-            sbase = a.s0 + (size_t)e * a.s_stride;
-            zbase = a.z0 + (size_t)e * a.s_stride;
-        }
-        bsrc[i] = wbase + (size_t)grow * KT * kTileBytes + (size_t)lane * 16;
-        const size_t so = (size_t)(grow * kTileRows + (lane & 15)) * NG;
-        ssrc[i] = reinterpret_cast<const f16*>(sbase) + so;
-        zsrc[i] = ZP ? reinterpret_cast<const f16*>(zbase) + so : nullptr;
-    }
-
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    for (int kt = 0; kt < KT; ++kt) {
-        // activations straight into LDS (fragment (msub, s) at ((msub * 4 + s) * 64 + lane) * 16 B)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            if (alive[i]) {
-                const int msub = wave + 4 * i;
-#pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    load_lds16(arow[i] + kt * kTileK + s * 32, As + (size_t)(msub * 4 + s) * kFragHalfs);
-            }
-        // weights: 16 bytes per lane per row block -> four exact f16 fragments
-        u32x4 wv[2];
-        f16 sc[2][4], zc[2][4];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            wv[i] = *reinterpret_cast<const u32x4*>(bsrc[i] + (size_t)kt * kTileBytes);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                sc[i][s] = ssrc[i][kt * GPT + ((s * GPT) >> 2)];
-                if constexpr (ZP) zc[i][s] = zsrc[i][kt * GPT + ((s * GPT) >> 2)];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int rbl = wave + 4 * i;
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-                *reinterpret_cast<f16x8*>(Bs + ((size_t)(rbl * 4 + s) * 64 + lane) * 8) =
-                    ZP ? dequant8z(wv[i][s], scale2(sc[i][s]), zc[i][s]) : dequant8(wv[i][s], scale2(sc[i][s]));
-        }
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            f16x8 af[4], bf[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                af[i] = *reinterpret_cast<const f16x8*>(As + ((size_t)((wm * 4 + i) * 4 + s) * 64 + lane) * 8);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                // GU: j = 0,1 gate row blocks 2wn, 2wn+1; j = 2,3 the matching up blocks
-                const int rbl = GU ? ((j < 2) ? (2 * wn + j) : (4 + 2 * wn + (j - 2))) : (4 * wn + j);
-                bf[j] = *reinterpret_cast<const f16x8*>(Bs + ((size_t)(rbl * 4 + s) * 64 + lane) * 8);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = mfma16(af[i], bf[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-
-    // epilogue: lane holds C[m = msub*16 + 4*(lane/16) + r][n = nsub*16 + lane%16]
-    bool ovf = false;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = (wm * 4 + i) * 16 + 4 * (lane >> 4) + r;
-            if (m >= rows) continue;
-            const size_t orow = (size_t)(slot0 + m) * a.n_rows;
-            if constexpr (GU) {
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int col = ntile * 64 + wn * 32 + j * 16 + (lane & 15);
-                    const float v = silu_mul_f(acc[i][j][r], acc[i][j + 2][r]);
-                    ovf |= f16_overflow(v);
-                    a.act_out[orow + col] = (f16)v;
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int col = ntile * kPreBN + wn * 64 + j * 16 + (lane & 15);
-                    ovf |= f16_overflow(acc[i][j][r]);
-                    a.y_out[orow + col] = (f16)acc[i][j][r];
-                }
-            }
-        }
-    }
-    report_f16_overflow(a.status, ovf);
-}
-
 // ---------------------------------------------------------------------------
-// Large-tile variant (K = 896 or 1280): 256 slots x 256 weight rows per
+// Large-tile kernel (K = 896 or 1280): 256 slots x 256 weight rows per
 // workgroup, v_mfma_f32_32x32x16_f16 (the faster gfx950 f16 MFMA shape).
 //   * the 4 waves stack along M (64 slots each) and each covers all 256 weight
 //     rows (8 32-row blocks, 256 accumulator registers), so every activation
@@ -260,13 +103,7 @@ constexpr int kRingAhead = 4;               // B fragments read ahead of their u
 constexpr int kRing = kRingAhead + 2;       // register ring size
 constexpr int lds_reads_after(int f) { return 63 - f < kRingAhead - 1 ? 63 - f : kRingAhead - 1; }
 
-// DW: unquantised experts (the reference's BF16 expert format, uploaded as
-// f16, row-major [rows][K], a.w_stride bytes per expert): the B fragments go
-// global -> LDS by 16-byte DMA, one k-tile ahead, in the same fragment order
-// (lane l of fragment (k-step, n-block): weight row n-block * 32 + l % 32,
-// columns k-step * 16 + 8 * (l / 32) ..), so there is no dequantisation and no
-// weight register; GPT and ZP are unused.
-template <int GPT, bool GU, int KT, bool ZP, bool DW = false>
+template <int GPT, bool GU, int KT, bool ZP>
 __global__ __launch_bounds__(256) void experts_prefill_big_kernel(ExpertArgs a) {
     // B fragments: [buffer][k-step 0..7][n-block 0..7][64 lanes][8 f16]
     __shared__ __attribute__((aligned(16))) f16 Bs[2][8 * kBigNB * kFragHalfs];
@@ -337,26 +174,6 @@ __global__ __launch_bounds__(256) void experts_prefill_big_kernel(ExpertArgs a) 
             const int n = wave * 16 + (lane & 15), q4 = lane >> 4;
             bdst0 = (uint32_t)((((q4 >> 1) * kBigNB + (n >> 5)) * 64 + (n & 31) + 32 * (q4 & 1)) * 16);
         }
-        // DW: this wave DMAs the fragments of n-blocks 2 * wave and 2 * wave + 1
-        // (all 8 k-steps); the lane's row of each and its first column
-        const f16* drow[2];
-        if constexpr (DW) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int n = (2 * wave + h) * 32 + (lane & 31);  // local weight row
-                const f16* base;
-                int grow;
-                if constexpr (GU) {
-                    base = reinterpret_cast<const f16*>((n < kBigBN / 2 ? a.w0 : a.w1) + (size_t)e * a.w_stride);
-                    grow = ntile * (kBigBN / 2) + (n & (kBigBN / 2 - 1));
-                } else {
-                    base = reinterpret_cast<const f16*>(a.w0 + (size_t)e * a.w_stride);
-                    grow = ntile * kBigBN + n;
-                }
-                drow[h] = base + (size_t)grow * K + 8 * (lane >> 5);
-            }
-        }
-
         // The k-tile pipeline keeps its own load schedule: every global load is
         // issued by inline asm at a fixed point and every wait is an explicit
         // vmcnt tied to the registers it guards. Left to itself the compiler sinks
@@ -370,7 +187,7 @@ __global__ __launch_bounds__(256) void experts_prefill_big_kernel(ExpertArgs a) 
         //     start of k-tile kt, staged into LDS during k-tile kt+1.
         // Issue order within k-tile kt: B(kt+2), then A(kt+1, ks) after k-step ks.
         constexpr int AK = JN;         // activation loads per k-step
-        constexpr int NB = DW ? 16 : (ZP ? 3 : 2) * UNITS;  // loads (DW: DMAs) per k-tile of weights
+        constexpr int NB = (ZP ? 3 : 2) * UNITS;  // loads per k-tile of weights
         u32x4 braw[2][UNITS];
         typename std::conditional<GPT == 4, u32x2, uint32_t>::type bscr[2][UNITS], bzr[2][UNITS];
         f16x8 areg[JN][8];
@@ -381,16 +198,6 @@ __global__ __launch_bounds__(256) void experts_prefill_big_kernel(ExpertArgs a) 
             for (int j = 0; j < JN; ++j) {
                 gload<kt * kTileK * 2 + ks * 32>(areg[j][ks], arow[j]);
             }
-        };
-        // DW: the 16 fragment DMAs of k-tile kt into buffer kt & 1
-        auto issue_bd = [&](auto ktc) {
-            constexpr int kt = decltype(ktc)::value;
-#pragma unroll
-            for (int ks = 0; ks < 8; ++ks)
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    load_lds16(drow[h] + kt * kTileK + ks * 16,
-                               reinterpret_cast<uint8_t*>(&Bs[kt & 1][0]) + (ks * kBigNB + 2 * wave + h) * 1024);
         };
         auto issue_b = [&](auto ktc) {
             constexpr int kt = decltype(ktc)::value;
@@ -455,32 +262,20 @@ __global__ __launch_bounds__(256) void experts_prefill_big_kernel(ExpertArgs a) 
 #pragma unroll
             for (int nb = 0; nb < kBigNB; ++nb) acc[j][nb] = f32x16{};
 
-        if constexpr (DW) {
-            // prologue: B(0) by DMA, A(0); B(0) landed in every wave's part
-            issue_bd(std::integral_constant<int, 0>{});
-            static_for<8>([&](auto ksc) { issue_a(std::integral_constant<int, 0>{}, ksc); });
-            vm_wait<8 * AK>();
-        } else {
-            // prologue: B(0), B(1), A(0); stage B(0)
-            issue_b(std::integral_constant<int, 0>{});
-            if constexpr (KT > 1) issue_b(std::integral_constant<int, 1>{});
-            static_for<8>([&](auto ksc) { issue_a(std::integral_constant<int, 0>{}, ksc); });
-            wait_b(std::integral_constant<int, (KT > 1 ? NB : 0) + 8 * AK>{}, 0);
-            static_for<UNITS>([&](auto ic) { static_for<4>([&](auto sc) { stage_run(0, ic, sc); }); });
-            lgkm_wait<0>();
-        }
+        // prologue: B(0), B(1), A(0); stage B(0)
+        issue_b(std::integral_constant<int, 0>{});
+        if constexpr (KT > 1) issue_b(std::integral_constant<int, 1>{});
+        static_for<8>([&](auto ksc) { issue_a(std::integral_constant<int, 0>{}, ksc); });
+        wait_b(std::integral_constant<int, (KT > 1 ? NB : 0) + 8 * AK>{}, 0);
+        static_for<UNITS>([&](auto ic) { static_for<4>([&](auto sc) { stage_run(0, ic, sc); }); });
+        lgkm_wait<0>();
         __syncthreads();
         static_for<KT>([&](auto ktc) {
             constexpr int kt = decltype(ktc)::value;
             constexpr bool more = kt + 1 < KT;
-            // weight loads issued after A(kt, *) and before A(kt + 1, *): DW the
-            // DMAs of B(kt + 1) (into the buffer the last k-tile read), else B(kt + 2)
-            constexpr int nB2 = DW ? (more ? NB : 0) : (kt + 2 < KT ? NB : 0);
-            if constexpr (DW) {
-                if constexpr (more) issue_bd(std::integral_constant<int, kt + 1>{});
-            } else {
-                if constexpr (kt + 2 < KT) issue_b(std::integral_constant<int, kt + 2>{});
-            }
+            // weight loads issued after A(kt, *) and before A(kt + 1, *): B(kt + 2)
+            constexpr int nB2 = kt + 2 < KT ? NB : 0;
+            if constexpr (kt + 2 < KT) issue_b(std::integral_constant<int, kt + 2>{});
             // B fragments stream from LDS through a 6-deep register ring, read
             // 4 fragments (8 MFMAs) ahead of their use: fragment f = ks * 8 + nb
             const uint32_t bb = lds_addr(Bs[kt & 1]) + lane * 16;
@@ -502,15 +297,13 @@ __global__ __launch_bounds__(256) void experts_prefill_big_kernel(ExpertArgs a) 
                 // every third fragment from fragment 8 on, so the VALU work
                 // interleaves with the MFMAs in flight
                 constexpr int run = (f - 8) / 3;
-                if constexpr (!DW && more && f >= 8 && (f - 8) % 3 == 0 && run < 4 * UNITS) {
+                if constexpr (more && f >= 8 && (f - 8) % 3 == 0 && run < 4 * UNITS) {
                     // B(kt+1) was issued before A(kt), B(kt+2) and A(kt+1, 0)
                     if constexpr (run == 0) wait_b(std::integral_constant<int, 8 * AK + nB2 + AK>{}, (kt + 1) & 1);
                     stage_run(kt + 1, std::integral_constant<int, run / 4>{}, std::integral_constant<int, run % 4>{});
                 }
             });
             lgkm_wait<0>();  // this k-tile's staging writes (asm, not tracked by the compiler)
-            // DW: B(kt + 1)'s DMAs, older than A(kt + 1, *), have landed
-            if constexpr (DW && more) vm_wait<8 * AK>();
             __syncthreads();
         });
 
@@ -592,26 +385,14 @@ static bool launch_big(const ExpertArgs& a, int max_tiles, hipStream_t st) {
 
 template <bool GU, bool ZP>
 static hipError_t launch_prefill_g(const ExpertArgs& a, int max_tiles, hipStream_t st) {
-    const int n_ntiles = GU ? (a.n_rows / (kPreBN / 2)) : (a.n_rows / kPreBN);
-    const dim3 grid(max_tiles * n_ntiles);
-    if (a.bm == kBigBM) {
-        bool done = false;
-        switch (a.group) {
-            case 32: done = launch_big<4, GU, ZP>(a, max_tiles, st); break;
-            case 64: done = launch_big<2, GU, ZP>(a, max_tiles, st); break;
-            case 128: done = launch_big<1, GU, ZP>(a, max_tiles, st); break;
-            default: return hipErrorInvalidValue;
-        }
-        return done ? hipGetLastError() : hipErrorInvalidValue;
-    }
-    if (a.bm != kPreBM) return hipErrorInvalidValue;
+    bool done = false;
     switch (a.group) {
-        case 32: launch_k((experts_prefill_kernel<4, GU, ZP>), grid, dim3(256), 0, st, a); break;
-        case 64: launch_k((experts_prefill_kernel<2, GU, ZP>), grid, dim3(256), 0, st, a); break;
-        case 128: launch_k((experts_prefill_kernel<1, GU, ZP>), grid, dim3(256), 0, st, a); break;
+        case 32: done = launch_big<4, GU, ZP>(a, max_tiles, st); break;
+        case 64: done = launch_big<2, GU, ZP>(a, max_tiles, st); break;
+        case 128: done = launch_big<1, GU, ZP>(a, max_tiles, st); break;
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
+    return done ? hipGetLastError() : hipErrorInvalidValue;
 }
 
 }  // namespace uocr_hip

@@ -192,7 +192,8 @@ hipError_t launch_decode_stream(const DecodeArgs& a, hipStream_t st);
 
 hipError_t launch_router(const RouterArgs& a, bool x_is_bf16, hipStream_t st);
 constexpr int kDecodeTileRows = 16;
-constexpr int kPrefillTileRows = 128;     // generic prefill kernel
+constexpr int kPrefillSmallTileRows = 64;  // the tiles of int4_tile_kernel
+constexpr int kPrefillTileRows = 128;
 constexpr int kPrefillBigTileRows = 256;  // large-tile prefill kernel (K in {896, 1280})
 // the large-tile kernel is instantiated for 7 and 10 k-tiles and tiles its
 // output in 128 act columns (gate/up) and 256 hidden columns (down)
@@ -210,7 +211,6 @@ constexpr size_t kGroupScanLds = 96 * 1024;  // per-(chunk, expert) counts of th
 bool group_fits(int seq, int top_k, int n_experts);  // the grouping scan's LDS holds seq * top_k entries
 hipError_t router_overflow_read(int clear, int* flag);  // sticky count > cap flag of the router mirror
 hipError_t launch_experts_prefill(const ExpertArgs& a, bool gate_up, int max_tiles, hipStream_t st);
-hipError_t launch_experts_prefill_dense(const ExpertArgs& a, bool gate_up, int max_tiles, hipStream_t st);
 hipError_t launch_combine(const CombineArgs& c, hipStream_t st);
 
 // Unquantised (bf16 / f32 checkpoint) matrices held as f16 row-major
