@@ -57,6 +57,7 @@ struct MirrorArgs {
     int cap;
     int K, N, group;
     int m_plain;  // plain GEMM: rows of x
+    int n_experts, n_z;  // experts (plain: 1); workgroups per (column block, expert)
     float* out;   // gate/up: act [E, cap, N]; down: out [T, N] (+=); plain: y [m, N]
 };
 
@@ -69,15 +70,22 @@ __global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
     __shared__ __attribute__((aligned(16))) f16 As[16 * kMFrag];
     __shared__ __attribute__((aligned(16))) f16 Bs[NM * 16 * kMFrag];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int e = MODE == kPlain ? 0 : blockIdx.y;
-    const int n0 = blockIdx.x * kMBN;
+    // Block b runs on XCD b % 8. Grouped: every column block of an expert on one
+    // XCD, so its gathered f32 rows (read once per column block) stay in that L2;
+    // plain: every column block of an m-tile.
+    const int nbx = a.N / kMBN, local = blockIdx.x >> 3;
+    const int n0 = local % nbx * kMBN, rest = local / nbx;
+    const int n_e8 = (a.n_experts + 7) / 8;
+    const int e = MODE == kPlain ? 0 : rest % n_e8 * 8 + (blockIdx.x & 7);
+    const int z = MODE == kPlain ? rest * 8 + (blockIdx.x & 7) : rest / n_e8;
+    if (e >= a.n_experts || z >= a.n_z) return;
     const int rows = MODE == kPlain ? a.m_plain : min(a.count[e], a.cap);
     const int K = a.K, N = a.N;
     const int packed_row = (K + 1) / 2;
 
-    // m-tiles blockIdx.z, + gridDim.z, ...: a skewed expert's rows spread over
-    // gridDim.z workgroups per column block
-    for (int m0 = blockIdx.z * kMBM; m0 < rows; m0 += gridDim.z * kMBM) {
+    // m-tiles z, + n_z, ...: a skewed expert's rows spread over n_z workgroups
+    // per column block
+    for (int m0 = z * kMBM; m0 < rows; m0 += a.n_z * kMBM) {
         f32x4 acc[NM][4];
 #pragma unroll
         for (int j = 0; j < NM; ++j)
@@ -136,17 +144,21 @@ __global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
                 }
             }
         };
+        const u32x4 zero4 = {0u, 0u, 0u, 0u};
+        auto masked = [&](f16x8 v, bool on) {
+            return __builtin_bit_cast(f16x8, on ? __builtin_bit_cast(u32x4, v) : zero4);
+        };
         auto store = [&](int kc) {
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
                 const int m = (tid + 256 * it) >> 4;
-                const bool on = alive[it] && c8 * 8 < kc;
                 f16x8 v;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    v[i] = on ? (f16)ar[it][0][i] : (f16)0.0f;
-                    v[4 + i] = on ? (f16)ar[it][1][i] : (f16)0.0f;
+                    v[i] = (f16)ar[it][0][i];
+                    v[4 + i] = (f16)ar[it][1][i];
                 }
+                v = masked(v, alive[it] && c8 * 8 < kc);
                 // fragment (m / 16, k-step c8 / 4), lane (m % 16) + 16 * (c8 % 4)
                 const int frag = (m >> 4) * 4 + (c8 >> 2);
                 *reinterpret_cast<f16x8*>(As + (size_t)frag * kMFrag + ((m & 15) + 16 * (c8 & 3)) * 8) = v;
@@ -164,8 +176,9 @@ __global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
 #pragma unroll
                         for (int i = 0; i < 8; ++i) {
                             const float q = (float)((w[r8] >> (4 * i)) & 0xfu);
-                            v[i] = on ? (f16)((q - zr[it]) * sr[it]) : (f16)0.0f;
+                            v[i] = (f16)((q - zr[it]) * sr[it]);
                         }
+                        v = masked(v, on);
                         const int frag = (it * 4 + (n >> 4)) * 4 + c32;
                         *reinterpret_cast<f16x8*>(Bs + (size_t)frag * kMFrag + ((n & 15) + 16 * r8) * 8) = v;
                     }
@@ -179,9 +192,10 @@ __global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
                     f16x8 v;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        v[2 * i] = on ? (f16)bf16_bits_to_f32(w[i] & 0xffffu) : (f16)0.0f;
-                        v[2 * i + 1] = on ? (f16)__uint_as_float(w[i] & 0xffff0000u) : (f16)0.0f;
+                        v[2 * i] = (f16)bf16_bits_to_f32(w[i] & 0xffffu);
+                        v[2 * i + 1] = (f16)__uint_as_float(w[i] & 0xffff0000u);
                     }
+                    v = masked(v, on);
                     const int frag = (mat * 4 + (n >> 4)) * 4 + (c8 >> 2);
                     *reinterpret_cast<f16x8*>(Bs + (size_t)frag * kMFrag + ((n & 15) + 16 * (c8 & 3)) * 8) = v;
                 }
@@ -238,9 +252,12 @@ hipError_t launch_mirror(const MirrorArgs& a, int n_experts, hipStream_t st) {
     // m-tile workgroups per (column block, expert): every m-tile of a plain
     // GEMM; up to 32 per expert of the grouped calls (cap bounds the rows)
     const int mt = ((MODE == kPlain ? a.m_plain : a.cap) + kMBM - 1) / kMBM;
-    const int mz = MODE == kPlain ? std::min(mt, 65535) : std::min(mt, 32);
-    const dim3 grid(a.N / kMBN, MODE == kPlain ? 1 : n_experts, std::max(mz, 1));
-    launch_k((mirror_kernel<MODE, WFMT>), grid, dim3(256), 0, st, a);
+    MirrorArgs b = a;
+    b.n_experts = MODE == kPlain ? 1 : n_experts;
+    b.n_z = std::max(1, MODE == kPlain ? std::min(mt, 65535) : std::min(mt, 32));
+    const long long units = MODE == kPlain ? (b.n_z + 7) / 8 : (long long)((n_experts + 7) / 8) * b.n_z;
+    const dim3 grid((unsigned)(8 * units * (a.N / kMBN)));
+    launch_k((mirror_kernel<MODE, WFMT>), grid, dim3(256), 0, st, b);
     return hipGetLastError();
 }
 
