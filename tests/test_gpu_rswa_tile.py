@@ -101,3 +101,65 @@ def test_one_cache_tiles(dev, seq, q_start, kv_len, causal):
                                              causal, ptr(out), None))
         torch.cuda.synchronize()
         assert np.abs(out.cpu().numpy().reshape(seq, -1) - want).max() <= TOL, devlen
+
+
+@pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
+def test_keys_past_the_limit_are_not_used(dev, hd, heads, kv_heads):
+    """Rows of the cache past each request's length hold NaN and inf: the last
+    key block's tail must not reach the output (a weight of 0 times NaN would)."""
+    torch = _torch()
+    rng = np.random.default_rng(hd)
+    lens, cap = [97, 130, 33], 200
+    n = len(lens)
+    K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
+    for s, m in enumerate(lens):
+        K[s, m:], V[s, m:] = np.nan, np.inf
+    d_slots = np.concatenate([[s] * m for s, m in enumerate(lens)]).astype(np.int32)
+    d_pos = np.concatenate([np.arange(m) for m in lens]).astype(np.int32)
+    total = len(d_pos)
+    q = rand(rng, total, heads, hd)
+    out = torch.full((q.size,), float("nan"), dtype=torch.float32, device=dev)
+    print(f"[rswa tile] NaN past the limit hd={hd}", flush=True)
+    ok(lib().uocr_hip_rswa_attention_ragged(ptr(dev_f32(q, dev)), ptr(dev_f32(K, dev)), ptr(dev_f32(V, dev)),
+                                            ptr(dev_i32(d_slots, dev)), ptr(dev_i32(d_pos, dev)), total, cap, heads,
+                                            kv_heads, hd, ptr(out), None))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().reshape(total, heads * hd)
+    t0 = 0
+    for s, m in enumerate(lens):
+        want = O.rswa_attention(q[t0:t0 + m], K[s, :m], V[s, :m], m, 0, heads, kv_heads, hd, True).reshape(m, -1)
+        assert np.abs(got[t0:t0 + m] - want).max() <= TOL, s
+        t0 += m
+
+
+@pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
+def test_non_finite_values_stay_with_their_rows(dev, hd, heads, kv_heads):
+    """One request's V holds inf and NaN: the other requests' rows in the same
+    tiles, and its own rows before those positions, don't see them."""
+    torch = _torch()
+    rng = np.random.default_rng(hd + 1)
+    lens, cap = [97, 130, 33], 200
+    n = len(lens)
+    K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
+    V[1, 70, :, 3], V[1, 100] = np.inf, np.nan
+    d_slots = np.concatenate([[s] * m for s, m in enumerate(lens)]).astype(np.int32)
+    d_pos = np.concatenate([np.arange(m) for m in lens]).astype(np.int32)
+    total = len(d_pos)
+    q = rand(rng, total, heads, hd)
+    out = torch.full((q.size,), float("nan"), dtype=torch.float32, device=dev)
+    print(f"[rswa tile] inf and NaN values hd={hd}", flush=True)
+    ok(lib().uocr_hip_rswa_attention_ragged(ptr(dev_f32(q, dev)), ptr(dev_f32(K, dev)), ptr(dev_f32(V, dev)),
+                                            ptr(dev_i32(d_slots, dev)), ptr(dev_i32(d_pos, dev)), total, cap, heads,
+                                            kv_heads, hd, ptr(out), None))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().reshape(total, heads, hd)
+    t0 = 0
+    for s, m in enumerate(lens):
+        clean = 70 if s == 1 else m
+        want = O.rswa_attention(q[t0:t0 + clean], K[s, :clean], V[s, :clean], clean, 0, heads, kv_heads, hd,
+                                True).reshape(clean, heads, hd)
+        assert np.abs(got[t0:t0 + clean] - want).max() <= TOL, s
+        if s == 1:
+            assert not np.isfinite(got[t0 + 70:t0 + 100, :, 3]).any()
+            assert not np.isfinite(got[t0 + 100:t0 + m]).any()
+        t0 += m

@@ -61,195 +61,17 @@ struct RowLds {
     __attribute__((aligned(16))) float acc[WAVES][HDP];
 };
 
-// One (query row, head) by a workgroup of WAVES waves; keys split over
-// n_chunks calls (chunk = chunk).
 template <int HDP, int WAVES>
 __device__ __forceinline__ void row_attention(const RswaArgs& a, int row, int head, int chunk, RowLds<HDP, WAVES>& s) {
-    constexpr int D = HDP / 8;  // dims per lane
-    constexpr int NV = D / 4;   // float4 per lane per row
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int j = lane >> 3, p = lane & 7;
-    const int hd = a.head_dim, stride = a.kv_heads * hd;
-    const int kvh = head / (a.heads / a.kv_heads);
-    const float* kc = a.kc;
-    const float* vc = a.vc;
-    int limit;
-    if (a.mode <= 1) {
-        const int kv_len = a.mode == 1 ? *a.d_len : a.kv_len;
-        limit = a.causal ? min(kv_len, a.q_start + row + 1) : kv_len;
-    } else {
-        const int slot = a.d_slots[row];
-        limit = a.mode == 2 ? a.d_len[slot] : a.d_pos[row] + 1;
-        kc += (size_t)slot * a.batch_cap * stride;
-        vc += (size_t)slot * a.batch_cap * stride;
-    }
-    const size_t qoff = ((size_t)row * a.heads + head) * hd;
-    kc += (size_t)kvh * hd;
-    vc += (size_t)kvh * hd;
-    // lane p's dims: 4 at 4p + 32i (i < NV), so the 8 lanes of a key read one
-    // contiguous 128-byte run per load
-    auto dim_of = [&](int i) { return 4 * p + 32 * i; };
-
-    f32x4 qv[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-        qv[i] = dim_of(i) < hd ? *reinterpret_cast<const f32x4*>(a.q + qoff + dim_of(i)) : f32x4{0.f, 0.f, 0.f, 0.f};
-
-    float m = -INFINITY, l = 0.0f;
-    f32x4 acc[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // this workgroup's keys [kbeg, kend): chunk blockIdx.z of n_chunks (chunks
-    // of whole 8-key groups; a chunk past the limit has no keys)
-    int kbeg = 0, kend = limit;
-    if (a.n_chunks > 1) {
-        const int cs = ((limit + a.n_chunks - 1) / a.n_chunks + 7) & ~7;
-        kbeg = min(limit, chunk * cs);
-        kend = min(limit, kbeg + cs);
-    }
-    const int n_groups = (kend - kbeg + 7) / 8;
-    // Unpredicated loads (a lane-predicated load makes the compiler wait for
-    // every outstanding load before the first use, defeating the prefetch):
-    // keys past the limit re-read the last valid row (their weight is 0),
-    // dims past head_dim re-read the last 4 (their q is 0 and they are never
-    // stored). Called only with limit >= 1.
-    auto load = [&](int g, f32x4 (&kv)[NV], f32x4 (&vv)[NV]) {
-        const int t = min(kbeg + g * 8 + j, kend - 1);
-        const float* kr = kc + (size_t)t * stride;
-        const float* vr = vc + (size_t)t * stride;
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int d = min(dim_of(i), hd - 4);
-            kv[i] = *reinterpret_cast<const f32x4*>(kr + d);
-            vv[i] = *reinterpret_cast<const f32x4*>(vr + d);
-        }
-    };
-    f32x4 k0[NV], v0[NV], k1[NV], v1[NV], k2[NV], v2[NV];
-    constexpr float kLog2e = 1.4426950408889634f;
-    auto step = [&](int g, const f32x4 (&kv)[NV], const f32x4 (&vv)[NV]) {
-        float part = 0.0f;
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) part = fmaf(qv[i][c], kv[i][c], part);
-        part += __shfl_xor(part, 1, 64);
-        part += __shfl_xor(part, 2, 64);
-        part += __shfl_xor(part, 4, 64);
-        const bool valid = kbeg + g * 8 + j < kend;
-        const float sc = valid ? part * a.scale : -INFINITY;
-        float mg = fmaxf(sc, __shfl_xor(sc, 8, 64));
-        mg = fmaxf(mg, __shfl_xor(mg, 16, 64));
-        mg = fmaxf(mg, __shfl_xor(mg, 32, 64));
-        const float m_new = fmaxf(m, mg);  // finite: key 0 of the group is valid
-        const float alpha = __builtin_amdgcn_exp2f((m - m_new) * kLog2e);
-        const float beta = valid ? __builtin_amdgcn_exp2f((sc - m_new) * kLog2e) : 0.0f;
-        float bs = beta + __shfl_xor(beta, 8, 64);
-        bs += __shfl_xor(bs, 16, 64);
-        bs += __shfl_xor(bs, 32, 64);
-        l = fmaf(l, alpha, bs);
-#pragma unroll
-        for (int i = 0; i < NV; ++i)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[i][c] = fmaf(acc[i][c], alpha, beta * vv[i][c]);
-        m = m_new;
-    };
-    // groups wave, wave + 8, ...; two groups' loads in flight beyond the one in
-    // use (three register buffers in rotation), one for head_dim > 128
-    constexpr int GS = WAVES;
-    int g = wave;
-    if constexpr (HDP <= 128) {
-        if (g < n_groups) {
-            load(g, k0, v0);
-            load(g + GS, k1, v1);
-        }
-        while (g < n_groups) {
-            load(g + 2 * GS, k2, v2);
-            step(g, k0, v0);
-            g += GS;
-            if (g >= n_groups) break;
-            load(g + 2 * GS, k0, v0);
-            step(g, k1, v1);
-            g += GS;
-            if (g >= n_groups) break;
-            load(g + 2 * GS, k1, v1);
-            step(g, k2, v2);
-            g += GS;
-        }
-    } else {
-        if (g < n_groups) load(g, k0, v0);
-        while (g < n_groups) {
-            load(g + GS, k1, v1);
-            step(g, k0, v0);
-            g += GS;
-            if (g >= n_groups) break;
-            load(g + GS, k0, v0);
-            step(g, k1, v1);
-            g += GS;
-        }
-    }
-    // sum the 8 key slots of the wave (same m within the wave)
-#pragma unroll
-    for (int i = 0; i < NV; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            float x = acc[i][c];
-            x += __shfl_xor(x, 8, 64);
-            x += __shfl_xor(x, 16, 64);
-            x += __shfl_xor(x, 32, 64);
-            acc[i][c] = x;
-        }
-    auto& wm = s.m;
-    auto& wl = s.l;
-    auto& wacc = s.acc;
-    if (lane < 8) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) *reinterpret_cast<f32x4*>(&wacc[wave][dim_of(i)]) = acc[i];
-    }
-    if (lane == 0) {
-        wm[wave] = m;
-        wl[wave] = l;
-    }
-    __syncthreads();
-    // combine the waves (a wave without keys has m = -inf and weight 0)
-    float* rec = a.n_chunks > 1 ? a.part + (((size_t)row * a.heads + head) * a.n_chunks + chunk) * kRswaRec
-                                : nullptr;
-    if (rec && tid == 0) {
-        float M = -INFINITY, L = 0.0f;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, wm[w]);
-        if (M != -INFINITY) {
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w)
-                L = fmaf(wl[w], wm[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((wm[w] - M) * kLog2e), L);
-        }
-        rec[0] = M;
-        rec[1] = L;
-    }
-    for (int d = tid; d < hd; d += WAVES * 64) {
-        float M = -INFINITY;
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, wm[w]);
-        float L = 0.0f, o = 0.0f;
-        if (M != -INFINITY) {
-#pragma unroll
-            for (int w = 0; w < WAVES; ++w) {
-                const float f = wm[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((wm[w] - M) * kLog2e);
-                L = fmaf(wl[w], f, L);
-                o = fmaf(wacc[w][d], f, o);
-            }
-        }
-        if (rec)
-            rec[4 + d] = o;  // unnormalised, relative to this chunk's max
-        else
-            a.out[qoff + d] = L > 0.0f ? o / L : 0.0f;
-    }
+#include "rswa_row_body.hpp"
 }
 
 template <int HDP>
 __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
-    __shared__ RowLds<HDP, kRswaWaves> s;
-    row_attention<HDP, kRswaWaves>(a, blockIdx.x, blockIdx.y, blockIdx.z, s);
+    constexpr int WAVES = kRswaWaves;
+    __shared__ RowLds<HDP, WAVES> s;
+    const int row = blockIdx.x, head = blockIdx.y, chunk = blockIdx.z;
+#include "rswa_row_body.hpp"
 }
 
 // ---------------------------------------------------------------------------
@@ -360,6 +182,7 @@ struct TileLds {
         __attribute__((aligned(16))) float q[32 * HD];
         struct {  // once the last scores are done
             float m[kTileWaves][32], l[kTileWaves][32];
+            int redo;
         };
     };
 };
@@ -381,7 +204,7 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
     };
     __shared__ Lds s;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (scalar: it is in the loads' scalar offsets)
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (scalar: the loads' offsets and buffers are)
     const int i = lane & 31, h = lane >> 5;
     int slot, limit;
     if ((int)blockIdx.x >= n_tiles * a.heads) {  // row worker: the rows of the tiles that don't pay
@@ -462,8 +285,9 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
         const int mylim = in ? limit : 0;
         const int kend = __builtin_amdgcn_readfirstlane(half_max(mylim));
         const size_t base = (a.mode == 3 ? (size_t)ps * a.batch_cap * stride : 0) + (size_t)kvh * HD;
-        // buffer loads: keys past kend are out of range and read as zeros
-        // (base + kvh * HD: the last key's row ends before the next key's)
+        // buffer loads: keys past kend are out of range and read as zeros (base
+        // + kvh * HD: the last key's row ends before the next key's). The key's
+        // offset is in the vector offset, which alone is certain to be checked against the size.
         const int bytes = ((kend - 1) * stride + HD) * 4, rowb = stride * 4;
         const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.kc + base), 0, bytes, 0x00020000);
         const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.vc + base), 0, bytes, 0x00020000);
@@ -479,7 +303,7 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
             for (int n = 0; n < U / 2; ++n)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(
                     kr, (__attribute__((address_space(3))) void*)(kbuf + n * 256), 16,
-                    kvo + (ku ^ ((n * (64 / U)) % U << 4)), (blk * 32 + n * (64 / U)) * rowb, 0, 0);
+                    kvo + (ku ^ ((n * (64 / U)) % U << 4)) + (blk * 32 + n * (64 / U)) * rowb, 0, 0, 0);
         };
         const int vvo = 4 * h * rowb + NB * i * 4;
         if (wave < nblk) load_k(wave);
@@ -494,11 +318,11 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
                 for (int r = 0; r < 8; ++r) {
                     const int so = (blk * 32 + 16 * half + 8 * (r >> 2) + (r & 3)) * rowb;
                     if constexpr (NB == 4) {
-                        const f32x4 t = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, vvo, so, 0));
+                        const f32x4 t = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, vvo + so, 0, 0));
 #pragma unroll
                         for (int b = 0; b < 4; ++b) v[half][r][b] = t[b];
                     } else {
-                        const u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(vr, vvo, so, 0));
+                        const u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(vr, vvo + so, 0, 0));
 #pragma unroll
                         for (int b = 0; b < 2; ++b) v[half][r][b] = __uint_as_float(t[b]);
                     }
@@ -581,6 +405,7 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
     // own K buffer (unit permuted by the query), then every thread sums
     l += __shfl_xor(l, 32, 64);
     __syncthreads();  // the query rows' place takes m and l
+    if (tid == 0) s.t.redo = 0;
     if (h == 0) {
         s.t.m[wave][i] = m;
         s.t.l[wave][i] = l;
@@ -598,6 +423,7 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
     __syncthreads();
     for (int u = tid; u < 32 * 32; u += kTileWaves * 64) {
         const int qi = u / 32, rho = u % 32, row = tile * kTileQ + qi;
+        const int row_keys = __shfl(limit, qi, 64);
         if (row >= rows) continue;
         float M = -INFINITY, L = 0.0f, acc[NB] = {};
 #pragma unroll
@@ -612,8 +438,25 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
             }
         }
         float* op = a.out + ((size_t)row * a.heads + head) * HD + NB * rho;
+        bool finite = L > 0.0f && L < INFINITY;
 #pragma unroll
-        for (int b = 0; b < NB; ++b) op[b] = L > 0.0f ? acc[b] / L : 0.0f;
+        for (int b = 0; b < NB; ++b) {
+            op[b] = L > 0.0f ? acc[b] / L : 0.0f;
+            finite &= fabsf(acc[b]) < INFINITY;
+        }
+        if (row_keys > 0 && !finite) s.t.redo = 1;
+    }
+    // An infinite or NaN value meets a weight of 0 in the rows of the tile that
+    // do not see its key (another request's, a later position's): such a tile
+    // is done again row by row, where every row reads its own keys only.
+    __syncthreads();
+    const int redo = s.t.redo;
+    __syncthreads();  // (the rows' results take its place)
+    if (redo) {
+        for (int r = 0; r < min(kTileQ, rows - tile * kTileQ); ++r) {
+            row_attention<HD, kTileWaves>(a, tile * kTileQ + r, head, 0, s.r);
+            __syncthreads();
+        }
     }
 }
 
@@ -751,8 +594,7 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
     float* part = nullptr;
     int cus = 0;
     const long long wgs = (long long)rows * a.heads;
-    const bool known = rswa_device(&part, &cus) == 0;
-    if (wgs < 512 && known) {
+    if (wgs < 512 && rswa_device(&part, &cus) == 0) {
         int n = (int)((2LL * cus + wgs - 1) / wgs);
         if (max_len > 0) n = std::min(n, max_len / 128);
         n = std::min(n, 8);
@@ -772,7 +614,7 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
         wgs * (max_len > 0 ? max_len : 128) >= kTileMinWork) {
         const int n_tiles = (rows + kTileQ - 1) / kTileQ;
         const dim3 tgrid(n_tiles * a.heads + (int)std::min<long long>(wgs, kRowWorkers));
-        const bool sort = n_tiles * a.heads > 2 * cus;
+        const bool sort = n_tiles * a.heads > 512;  // (two workgroups on each of 256 CUs)
         if (a.head_dim == 64) launch_k(rswa_tile_kernel<64>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
         else launch_k(rswa_tile_kernel<128>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
         const hipError_t te = hipGetLastError();
