@@ -247,7 +247,7 @@ def run_config(cfg, steps, warmup, replicas, group=32, graph=False, fmt="int4"):
             res["gate_up_mfma_frac"] = res["gate_up_tflops"] / MFMA_PEAK_TFLOPS
             if getattr(layers_np[0], "gate_w", None) is not None:  # bf16 experts (dense.hip)
                 big = seq >= 256
-                res["dominant"] = {"kernel": "dense_tiled_kernel<true> (gate+up)" if big else
+                res["dominant"] = {"kernel": f"dense_tile_kernel<{64 if seq * layers_np[0].top_k <= 56 * layers_np[0].n_experts else 128}, true, 2> (gate+up)" if big else
                                    "dense_skinny_kernel<4, 10, true, 0> (gate+up)", "ms": stage["gate_up"],
                                    "bytes": avg["gate_up"], "gbs": res["gate_up_gbs"], "flops": fl_gu,
                                    "tflops": res["gate_up_tflops"], "mfma_frac": res["gate_up_mfma_frac"],
@@ -489,9 +489,9 @@ def run_rswa_prefill(steps, warmup, batch=4, rows=1000, heads=10, kv_heads=10, h
     pairs = batch * rows * (rows + 1) // 2
     flops = 4.0 * head_dim * heads * pairs
     return {"workload": f"rswa_prefill_ragged_{batch}x{rows}_h{heads}_d{head_dim}", "ms_per_step": ms,
-            "kernel": "rswa_kernel (uocr_hip_rswa_attention_ragged)", "flops": flops,
+            "kernel": "rswa_tile_kernel<128> (uocr_hip_rswa_attention_ragged)", "flops": flops,
             "tflops": flops / (ms * 1e-3) / 1e12,
-            "note": "f32 VALU online softmax, one workgroup per (row, head); no MFMA query tiling"}
+            "note": "f32 MFMA, 32 query rows per workgroup"}
 
 
 def run_rswa(steps, warmup, batch=16, prefill=1000, window=128, heads=10, kv_heads=10, head_dim=128, replicas=2):

@@ -19,6 +19,12 @@
 // Epilogues: gate/up -> silu(g) * u into act [E, cap, N] (cpu_ops.cpp:108-113);
 // down -> out[token] += w * y with f32 atomics (the reference's scatter-add,
 // moe_device.cu:261-266; the order of the adds is not fixed); plain GEMM -> y.
+// Bound by the staging: every m-tile dequantises its panel again and gathers f32
+// rows, so a chunk's loads are issued into registers under the previous chunk's
+// MFMAs, and the grid puts the column blocks of one expert on one XCD (its rows
+// then come from one L2). Measured at 1024 tokens, 64 experts, top-6 (rocprofv3):
+// gate/up 152 -> 131 us, down 108 -> 82, matmul_t_bf16 38 -> 33. Not faster:
+// 128-row m-tiles (gate/up 154), loads two chunks ahead.
 #include "launch.hpp"
 
 #include <algorithm>
