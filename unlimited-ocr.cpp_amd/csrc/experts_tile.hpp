@@ -233,7 +233,14 @@ __global__ __launch_bounds__(256, 2) void int4_tile_kernel(ExpertArgs a, int n_t
         step(t2, C1{}, C2{});
         if (++t2 == KT2) break;
     }
-    vm_wait<0>();  // no DMA may outlive the workgroup's LDS
+    // The last step's weight loads (repeats of the last tile) have no use: they are
+    // waited for while their registers are still theirs, or one that lands later
+    // would overwrite what the epilogue holds in them. No DMA may outlive the
+    // workgroup's LDS either.
+    vm_wait<0>();
+    tie_b(C0{});
+    tie_b(C1{});
+    tie_b(C2{});
 
     // D lane l: weight row 8 * (r / 4) + 4 * (l / 32) + r % 4 of the block, slot l % 32
     bool ovf = false;
