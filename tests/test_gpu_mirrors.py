@@ -284,3 +284,65 @@ def test_host_grouping_branch_from_mirrors(dev, seq):
     ops.add_scaled(out, so, 1.0)
     torch.cuda.synchronize()
     _check(out.cpu().numpy(), want, f"host-grouping-mirrors-t{seq}")
+
+
+@pytest.mark.parametrize("fmt", ["int4", "bf16"])
+@pytest.mark.parametrize("counts,cap", [
+    ([200], 200),                                     # one expert
+    ([0, 1, 64, 65, 0, 128, 300, 190], 192),          # tile edges, none, more than cap
+    ([3] * 63 + [0, 70, 5, 0, 64, 65, 1], 70),        # a second scan of 64 experts
+    ([320] * 12, 320),                                # more tiles than the grid has workgroups for
+])
+def test_grouped_tile_order(dev, fmt, counts, cap):
+    """(m-tile, column block) items of any expert count and skew, against the
+    definition in 64 bits. Bar: operands rounded to f16 (2^-11 each) and f32 sums:
+    2e-3 relative."""
+    import torch
+    from uocr_hip import ops, synth
+    rng = np.random.default_rng(len(counts))
+    E, T, H, I = len(counts), 256, 192, 128
+    n = np.minimum(counts, cap)
+    x = rng.standard_normal((T, H)).astype(np.float32)
+    tok = np.full((E, cap), -1, np.int32)
+    for e in range(E):
+        tok[e, : n[e]] = rng.integers(0, T, n[e])
+    tw = rng.uniform(0.1, 1.0, (E, cap)).astype(np.float32)
+    xt, tt, twt, ct = (torch.from_numpy(a).to(dev) for a in (x, tok, tw, np.asarray(counts, np.int32)))
+    act = torch.zeros(E, cap, I, device=dev)
+    out = torch.zeros(T, H, device=dev)
+    print(f"[mirror] tile order {fmt} E={E}", flush=True)
+    if fmt == "int4":
+        g, u, d = ([synth.random_qmat(rng, r, c, 32, 0.02) for _ in range(E)] for r, c in ((I, H), (I, H), (H, I)))
+        wg, wu, wd = ([q.dequantize().astype(np.float64) for q in m] for m in (g, u, d))
+        gt, ut, dt = (ops.RefInt4Table(m, dev) for m in (g, u, d))
+        ops.moe_grouped_gate_up_int4(xt, gt, ut, tt, ct, cap, act)
+        ops.moe_grouped_down_int4(act, dt, tt, twt, ct, cap, out)
+    else:
+        g, u, d = ([synth.random_dense_bf16(rng, r, c, 0.1) for _ in range(E)] for r, c in ((I, H), (I, H), (H, I)))
+        wg, wu, wd = ([q.to_f32().astype(np.float64) for q in m] for m in (g, u, d))
+        gt, ut, dt = ([torch.from_numpy(q.data.view(np.int16)).to(dev) for q in m] for m in (g, u, d))
+        keep = ops.moe_grouped_gate_up_bf16(xt, gt, ut, tt, ct, cap, act)
+        keep = keep, ops.moe_grouped_down_bf16(act, dt, tt, twt, ct, cap, out)
+    torch.cuda.synchronize()
+    want = np.zeros((T, H))
+    for e in range(E):
+        xe = x[tok[e, : n[e]]].astype(np.float64)
+        a = xe @ wg[e].T
+        a = a / (1 + np.exp(-a)) * (xe @ wu[e].T)
+        assert rel_l2(act[e, : n[e]].cpu().numpy(), a) <= 2e-3 or n[e] == 0, e
+        np.add.at(want, tok[e, : n[e]], tw[e, : n[e], None] * (a @ wd[e].T))
+    assert rel_l2(out.cpu().numpy(), want) <= 2e-3
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 64, 96), (64, 3840, 128), (65, 3840, 160), (200, 64, 32), (449, 192, 256)])
+def test_matmul_tile_order(dev, m, n, k):
+    """Few and many column blocks, both item orders. Bar as above."""
+    import torch
+    from uocr_hip import ops, synth
+    rng = np.random.default_rng(m + n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    w = synth.random_dense_bf16(rng, n, k, 0.1)
+    y = torch.full((m, n), float("nan"), device=dev)
+    ops.matmul_t_bf16(torch.from_numpy(x).to(dev), torch.from_numpy(w.data.view(np.int16)).to(dev), y)
+    torch.cuda.synchronize()
+    assert rel_l2(y.cpu().numpy(), x.astype(np.float64) @ w.to_f32().astype(np.float64).T) <= 2e-3

@@ -6,8 +6,8 @@
 // or bf16 row-major matrices behind device pointer arrays, the [n_experts, cap]
 // assignment tables of moe_router_topk, f32 activations in and out.
 //
-// One kernel family serves every call: a workgroup owns (64 output rows, one
-// expert) and walks the expert's assigned rows in m-tiles of 64. Per 128-column
+// One kernel family serves every call: a workgroup takes 64 output rows of an m-tile
+// (64 assigned rows of one expert). Per 128-column
 // k-chunk it stages the gathered activation rows (f32 -> f16) and the weight
 // panel (INT4: (q - zero) * scale in f32, rounded once to f16, where the
 // reference dequantises to bf16, moe_gemm_int4.cu:456-473; bf16 weights:
@@ -21,11 +21,15 @@
 // moe_device.cu:261-266; the order of the adds is not fixed); plain GEMM -> y.
 // Bound by the staging: every m-tile dequantises its panel again and gathers f32
 // rows, so a chunk's loads are issued into registers under the previous chunk's
-// MFMAs, and the grid puts the column blocks of one expert on one XCD (its rows
-// then come from one L2). Measured at 1024 tokens, 64 experts, top-6 (rocprofv3):
-// gate/up 152 -> 131 us, down 108 -> 82, matmul_t_bf16 38 -> 33. Not faster:
-// 128-row m-tiles (gate/up 154), loads two chunks ahead.
+// MFMAs, and the grid gives each XCD an even run of (m-tile, column block) items. A whole
+// expert per XCD left most of the chip idle where few experts, or one m-tile of a
+// wide GEMM, hold the work: us, linear order without the register stage / expert per
+// XCD / this: matmul_t_bf16 1 row x 129280 x 1280 99 / 695 / 89, 1 x 3840 16.7 / 28.3 /
+// 16.4, gate/up of one expert at 512 rows 32 / 64 / 25, 64 experts with Zipf routing at
+// 1024 tokens 138 / 179 / 111, even 140 / 110 / 111. Not faster: 128-row m-tiles, loads
+// two chunks ahead.
 #include "launch.hpp"
+#include "xcd_order.hpp"
 
 #include <algorithm>
 
@@ -63,7 +67,7 @@ struct MirrorArgs {
     int cap;
     int K, N, group;
     int m_plain;  // plain GEMM: rows of x
-    int n_experts, n_z;  // experts (plain: 1); workgroups per (column block, expert)
+    int n_experts;  // (plain: unused)
     float* out;   // gate/up: act [E, cap, N]; down: out [T, N] (+=); plain: y [m, N]
 };
 
@@ -75,23 +79,55 @@ __global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
     // A: [4 m-subtiles][4 k-steps] fragments; B: [NM][4 n-subtiles][4 k-steps]
     __shared__ __attribute__((aligned(16))) f16 As[16 * kMFrag];
     __shared__ __attribute__((aligned(16))) f16 Bs[NM * 16 * kMFrag];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    // Block b runs on XCD b % 8. Grouped: every column block of an expert on one
-    // XCD, so its gathered f32 rows (read once per column block) stay in that L2;
-    // plain: every column block of an m-tile.
-    const int nbx = a.N / kMBN, local = blockIdx.x >> 3;
-    const int n0 = local % nbx * kMBN, rest = local / nbx;
-    const int n_e8 = (a.n_experts + 7) / 8;
-    const int e = MODE == kPlain ? 0 : rest % n_e8 * 8 + (blockIdx.x & 7);
-    const int z = MODE == kPlain ? rest * 8 + (blockIdx.x & 7) : rest / n_e8;
-    if (e >= a.n_experts || z >= a.n_z) return;
-    const int rows = MODE == kPlain ? a.m_plain : min(a.count[e], a.cap);
-    const int K = a.K, N = a.N;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int K = a.K, N = a.N, nbx = N / kMBN;
     const int packed_row = (K + 1) / 2;
 
-    // m-tiles z, + n_z, ...: a skewed expert's rows spread over n_z workgroups
-    // per column block
-    for (int m0 = z * kMBM; m0 < rows; m0 += a.n_z * kMBM) {
+    // m-tiles: the plain GEMM's, or every expert's in order (lane l holds expert
+    // base + l's count; each wave scans them itself)
+    auto tiles_of = [&](int e) { return e < a.n_experts ? (max(min(a.count[e], a.cap), 0) + kMBM - 1) / kMBM : 0; };
+    auto scan = [&](int v) {  // inclusive, over the wave
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(v, o, 64);
+            if (lane >= o) v += u;
+        }
+        return v;
+    };
+    int n_tiles = (a.m_plain + kMBM - 1) / kMBM, first64 = 0;
+    if constexpr (MODE != kPlain) {
+        first64 = tiles_of(lane);
+        n_tiles = 0;
+        for (int base = 0; base < a.n_experts; base += 64)
+            n_tiles += __shfl(scan(base ? tiles_of(base + lane) : first64), 63, 64);
+        n_tiles = __builtin_amdgcn_readfirstlane(n_tiles);
+    }
+
+    // Items (m-tile, column block), column blocks fastest: those of one m-tile share
+    // its f32 rows in one XCD's L2, and a popular expert's m-tiles are spread. A plain
+    // GEMM with fewer bytes of x than of W: m-tiles fastest, they share W's rows
+    // (448 rows, N 1280, K 1792: 26.6 us with column blocks fastest, 25.9)
+    const bool tile_fast = MODE == kPlain && 4ll * a.m_plain < (WFMT == 0 ? 1ll : 2ll) * N;
+    const int xcd = blockIdx.x % kXcds, last = xcd_first_item(xcd + 1, n_tiles * nbx);
+    for (int item = xcd_first_item(xcd, n_tiles * nbx) + blockIdx.x / kXcds; item < last; item += gridDim.x / kXcds) {
+        const int n0 = (tile_fast ? item / n_tiles : item % nbx) * kMBN;
+        int e = 0, m0 = (tile_fast ? item % n_tiles : item / nbx) * kMBM, rows = a.m_plain;
+        if constexpr (MODE != kPlain) {
+            int t = item / nbx;
+            for (int base = 0;; base += 64) {
+                const int inc = scan(base ? tiles_of(base + lane) : first64), all = __shfl(inc, 63, 64);
+                if (t < all) {
+                    const int k = __popcll(__ballot(inc <= t));
+                    e = base + k;
+                    if (k > 0) t -= __shfl(inc, k - 1, 64);
+                    break;
+                }
+                t -= all;
+            }
+            e = __builtin_amdgcn_readfirstlane(e);
+            m0 = __builtin_amdgcn_readfirstlane(t) * kMBM;
+            rows = min(a.count[e], a.cap);
+        }
         f32x4 acc[NM][4];
 #pragma unroll
         for (int j = 0; j < NM; ++j)
@@ -255,14 +291,13 @@ __global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
 
 template <int MODE, int WFMT>
 hipError_t launch_mirror(const MirrorArgs& a, int n_experts, hipStream_t st) {
-    // m-tile workgroups per (column block, expert): every m-tile of a plain
-    // GEMM; up to 32 per expert of the grouped calls (cap bounds the rows)
-    const int mt = ((MODE == kPlain ? a.m_plain : a.cap) + kMBM - 1) / kMBM;
+    // m-tiles that get workgroups of their own (more are looped over): a plain GEMM's,
+    // and of the grouped calls, whose counts the device knows, those of 8 experts per token
+    const long long mt = ((MODE == kPlain ? a.m_plain : a.cap) + kMBM - 1ll) / kMBM;
+    const long long tiles = MODE == kPlain ? mt : std::min(n_experts * mt, n_experts + 8 * mt);
     MirrorArgs b = a;
-    b.n_experts = MODE == kPlain ? 1 : n_experts;
-    b.n_z = std::max(1, MODE == kPlain ? std::min(mt, 65535) : std::min(mt, 32));
-    const long long units = MODE == kPlain ? (b.n_z + 7) / 8 : (long long)((n_experts + 7) / 8) * b.n_z;
-    const dim3 grid((unsigned)(8 * units * (a.N / kMBN)));
+    b.n_experts = n_experts;
+    const dim3 grid((unsigned)std::min((tiles * (a.N / kMBN) + kXcds - 1) / kXcds * kXcds, 1ll << 20));
     launch_k((mirror_kernel<MODE, WFMT>), grid, dim3(256), 0, st, b);
     return hipGetLastError();
 }
