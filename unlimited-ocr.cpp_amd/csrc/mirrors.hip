@@ -21,12 +21,13 @@
 // moe_device.cu:261-266; the order of the adds is not fixed); plain GEMM -> y.
 // Bound by the staging: every m-tile dequantises its panel again and gathers f32
 // rows, so a chunk's loads are issued into registers under the previous chunk's
-// MFMAs, and the grid gives each XCD an even run of (m-tile, column block) items. A whole
-// expert per XCD left most of the chip idle where few experts, or one m-tile of a
-// wide GEMM, hold the work: us, linear order without the register stage / expert per
-// XCD / this: matmul_t_bf16 1 row x 129280 x 1280 99 / 695 / 89, 1 x 3840 16.7 / 28.3 /
-// 16.4, gate/up of one expert at 512 rows 32 / 64 / 25, 64 experts with Zipf routing at
-// 1024 tokens 138 / 179 / 111, even 140 / 110 / 111. Not faster: 128-row m-tiles, loads
+// MFMAs, with the register count held to 3 (gate/up) or 4 workgroups per CU, and the
+// grid gives each XCD an even run of (m-tile, column block) items. A whole expert per
+// XCD left most of the chip idle where few experts, or one m-tile of a wide
+// GEMM, hold the work: us, linear order without the register stage / expert per XCD /
+// this: matmul_t_bf16 1 row x 129280 x 1280 99 / 695 / 86, 1 x 3840 16.7 / 28.3 / 15.6,
+// gate/up of one expert at 512 rows 32 / 64 / 23, 64 experts with Zipf routing at 1024
+// tokens 138 / 179 / 94, even 140 / 110 / 94. Not faster: 128-row m-tiles, loads
 // two chunks ahead.
 #include "launch.hpp"
 #include "xcd_order.hpp"
@@ -74,7 +75,7 @@ struct MirrorArgs {
 __device__ __forceinline__ float silu_mul_ref(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
 template <int MODE, int WFMT>
-__global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
+__global__ __launch_bounds__(256, MODE == kGateUp ? 3 : 4) void mirror_kernel(MirrorArgs a) {
     constexpr int NM = MODE == kGateUp ? 2 : 1;  // weight matrices
     // A: [4 m-subtiles][4 k-steps] fragments; B: [NM][4 n-subtiles][4 k-steps]
     __shared__ __attribute__((aligned(16))) f16 As[16 * kMFrag];
@@ -153,13 +154,14 @@ __global__ __launch_bounds__(256) void mirror_kernel(MirrorArgs a) {
         }
         const int c8 = tid & 15;
         constexpr int NW4 = WFMT == 0 ? NM : 4 * NM;  // 16-byte weight loads per thread
-        f32x4 ar[4][2];
+        f32x4 ar[4][2] = {};
         u32x4 wr[NW4];
         float sr[NM], zr[NM];  // INT4: a 32-column run lies in one group (group % 32 == 0)
         auto load = [&](int k0) {
             const int ka = min(k0 + c8 * 8, K - 8);
 #pragma unroll
             for (int it = 0; it < 4; ++it) {
+                if (m0 + 16 * it + 4 * wave >= rows) break;  // (this wave's rows of the rest: none)
                 ar[it][0] = *reinterpret_cast<const f32x4*>(arow[it] + ka);
                 ar[it][1] = *reinterpret_cast<const f32x4*>(arow[it] + ka + 4);
             }
