@@ -163,3 +163,29 @@ def test_non_finite_values_stay_with_their_rows(dev, hd, heads, kv_heads):
             assert not np.isfinite(got[t0 + 70:t0 + 100, :, 3]).any()
             assert not np.isfinite(got[t0 + 100:t0 + m]).any()
         t0 += m
+
+
+@pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
+def test_output_may_be_the_queries(dev, hd, heads, kv_heads):
+    """out == q, with inf and NaN values in reach of some rows (whose tiles are
+    partly done again): the same bits as with an output of its own."""
+    torch = _torch()
+    rng = np.random.default_rng(hd + 2)
+    lens, cap = [197, 230, 33], 300
+    n = len(lens)
+    K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
+    V[1, 70, :, 3], V[1, 100], K[0, 190] = np.inf, np.nan, np.nan
+    d_slots = dev_i32(np.concatenate([[s] * m for s, m in enumerate(lens)]).astype(np.int32), dev)
+    d_pos = dev_i32(np.concatenate([np.arange(m) for m in lens]).astype(np.int32), dev)
+    total = sum(lens)
+    q = dev_f32(rand(rng, total, heads, hd), dev)
+    out = torch.full_like(q, 7.0)
+    kc, vc = dev_f32(K, dev), dev_f32(V, dev)
+    print(f"[rswa tile] out == q hd={hd}", flush=True)
+    for dst in (out, q):
+        ok(lib().uocr_hip_rswa_attention_ragged(ptr(q), ptr(kc), ptr(vc), ptr(d_slots), ptr(d_pos), total, cap, heads,
+                                                kv_heads, hd, ptr(dst), None))
+    torch.cuda.synchronize()
+    a, b = out.cpu().numpy(), q.cpu().numpy()
+    assert np.array_equal(a, b, equal_nan=True)
+    assert not np.isfinite(a).all() and np.isfinite(a).mean() > 0.5

@@ -182,7 +182,7 @@ struct TileLds {
         __attribute__((aligned(16))) float q[32 * HD];
         struct {  // once the last scores are done
             float m[kTileWaves][32], l[kTileWaves][32];
-            int redo;
+            uint32_t redo;  // rows with a non-finite result
         };
     };
 };
@@ -438,25 +438,30 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
             }
         }
         float* op = a.out + ((size_t)row * a.heads + head) * HD + NB * rho;
-        bool finite = L > 0.0f && L < INFINITY;
+        bool bad = !(L > 0.0f && L < INFINITY);
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            op[b] = L > 0.0f ? acc[b] / L : 0.0f;
-            finite &= fabsf(acc[b]) < INFINITY;
+            acc[b] = L > 0.0f ? acc[b] / L : 0.0f;
+            bad |= !(fabsf(acc[b]) < INFINITY);
         }
-        if (row_keys > 0 && !finite) s.t.redo = 1;
+        // (a row's threads are one half of a wave)
+        if ((uint32_t)(__ballot(bad && row_keys > 0) >> (lane & 32))) {
+            if ((lane & 31) == 0) atomicOr(&s.t.redo, 1u << qi);
+        } else {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) op[b] = acc[b];
+        }
     }
     // An infinite or NaN value meets a weight of 0 in the rows of the tile that
-    // do not see its key (another request's, a later position's): such a tile
-    // is done again row by row, where every row reads its own keys only.
+    // do not see its key (another request's, a later position's): such rows are
+    // done again one by one, where every row reads its own keys only. Nothing
+    // of them is written before (out may be q).
     __syncthreads();
-    const int redo = s.t.redo;
+    uint32_t redo = __builtin_amdgcn_readfirstlane(s.t.redo);
     __syncthreads();  // (the rows' results take its place)
-    if (redo) {
-        for (int r = 0; r < min(kTileQ, rows - tile * kTileQ); ++r) {
-            row_attention<HD, kTileWaves>(a, tile * kTileQ + r, head, 0, s.r);
-            __syncthreads();
-        }
+    for (; redo; redo &= redo - 1) {
+        row_attention<HD, kTileWaves>(a, tile * kTileQ + __builtin_ctz(redo), head, 0, s.r);
+        __syncthreads();
     }
 }
 
