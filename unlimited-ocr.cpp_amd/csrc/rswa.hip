@@ -26,6 +26,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
+#include "rswa_dispatch.hpp"
 #include "uocr_hip/moe_capi.h"
 
 namespace uocr_hip {
@@ -108,7 +109,6 @@ constexpr int kTileSort = kTileWaves * 64;  // tiles that a call orders by their
 static_assert(kTileSort <= 256, "a tile's index has 8 bits of its sort key");
 constexpr int kTileCost = 4;      // row-blocks that a tile's key block costs
 constexpr int kRowWorkers = 512;  // at most
-constexpr long long kTileMinWork = 98304;
 
 // slot and key limit (rows attended, 0 past the end) of query row t
 __device__ __forceinline__ void row_limit(const RswaArgs& a, int rows, int t, int& slot, int& limit) {
@@ -609,14 +609,9 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
             a.part = part;
         }
     }
-    // One cache or ragged rows run query-tiled where the kernel is instantiated
-    // (head_dim 64 and 128), from kTileMinWork (row, head, key) triples, keys
-    // as far as the host knows them: below, the row kernel's shorter start
-    // wins (heads x rows x keys at head_dim 128, us against tiled: 600 x 60 13.1
-    // / 15.0, 970 x 60 15.6 / 19.2, 1630 x 60 23.6 / 24.1, 1300 x 130 23.7 / 17.6, 3000 x
-    // 300 57 / 26). Fewer than 512 pairs keep the key split above.
-    if (wgs >= 512 && a.mode != 2 && (a.head_dim == 64 || a.head_dim == 128) &&
-        wgs * (max_len > 0 ? max_len : 128) >= kTileMinWork) {
+    // One cache or ragged rows may run query-tiled (fewer than 512 pairs keep the
+    // key split above)
+    if (a.mode != 2 && rswa_call_tiled(rows, a.heads, a.head_dim, max_len)) {
         const int n_tiles = (rows + kTileQ - 1) / kTileQ;
         const dim3 tgrid(n_tiles * a.heads + (int)std::min<long long>(wgs, kRowWorkers));
         const bool sort = n_tiles * a.heads > 512;  // (two workgroups on each of 256 CUs)
