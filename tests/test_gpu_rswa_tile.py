@@ -189,3 +189,65 @@ def test_output_may_be_the_queries(dev, hd, heads, kv_heads):
     a, b = out.cpu().numpy(), q.cpu().numpy()
     assert np.array_equal(a, b, equal_nan=True)
     assert not np.isfinite(a).all() and np.isfinite(a).mean() > 0.5
+
+
+def _rows_want(q, K, V, slots, pos, heads, kv_heads, hd):
+    """Attention of every row over its slot's rows [0, pos], in 64 bits."""
+    T, cap = len(slots), K.shape[1]
+    q = q.reshape(T, heads, hd).astype(np.float64)
+    out = np.empty_like(q)
+    dead = np.arange(cap)[None] > pos[:, None]
+    for h in range(heads):
+        g = h // (heads // kv_heads)
+        s = np.einsum("td,tcd->tc", q[:, h], K[slots, :, g].astype(np.float64)) / np.sqrt(hd)
+        s[dead] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        out[:, h] = np.einsum("tc,tcd->td", p / p.sum(1, keepdims=True), V[slots, :, g].astype(np.float64))
+    return out.reshape(T, -1)
+
+
+@pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
+@pytest.mark.parametrize("name,lens,starts", [
+    ("one row each", [1] * 203, "any"),                        # row workers only, more than one row each
+    ("4 rows each", [4] * 60, 0), ("5 rows each", [5] * 45, 7),  # many passes: left to the workers
+    ("20 rows each", [20] * 14, 0),                            # few passes: tiles, a short last one
+    ("mixed", [1] * 70 + [130, 1, 9, 64, 2], "any"),           # both kinds in one call
+])
+def test_tiles_and_row_workers(dev, hd, heads, kv_heads, name, lens, starts):
+    """Every row is taken once, by a tile or by a worker, whatever the mix of requests."""
+    torch = _torch()
+    rng = np.random.default_rng(len(lens) + hd)
+    cap, n = 160, len(lens)
+    K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
+    first = [int(rng.integers(0, cap - m + 1)) if starts == "any" else starts for m in lens]
+    slots = np.concatenate([[s] * m for s, m in zip(rng.permutation(n), lens)]).astype(np.int32)
+    pos = np.concatenate([f + np.arange(m) for f, m in zip(first, lens)]).astype(np.int32)
+    total = len(pos)
+    q = rand(rng, total, heads, hd)
+    out = torch.full((q.size,), float("nan"), dtype=torch.float32, device=dev)
+    print(f"[rswa tile] {name} hd={hd}", flush=True)
+    ok(lib().uocr_hip_rswa_attention_ragged(ptr(dev_f32(q, dev)), ptr(dev_f32(K, dev)), ptr(dev_f32(V, dev)),
+                                            ptr(dev_i32(slots, dev)), ptr(dev_i32(pos, dev)), total, cap, heads,
+                                            kv_heads, hd, ptr(out), None))
+    torch.cuda.synchronize()
+    want = _rows_want(q, K, V, slots, pos, heads, kv_heads, hd)
+    assert np.abs(out.cpu().numpy().reshape(total, -1) - want).max() <= TOL
+
+
+def test_row_workers_past_256_tiles(dev):
+    """A call of more tiles than a worker looks at at once."""
+    torch = _torch()
+    rng = np.random.default_rng(8)
+    hd, heads, kv_heads, cap, total = 64, 2, 1, 5, 32 * 256 + 77
+    K, V = rand(rng, total, cap, kv_heads, hd), rand(rng, total, cap, kv_heads, hd)
+    slots = rng.permutation(total).astype(np.int32)
+    pos = rng.integers(0, cap, total).astype(np.int32)
+    q = rand(rng, total, heads, hd)
+    out = torch.full((q.size,), float("nan"), dtype=torch.float32, device=dev)
+    print("[rswa tile] past 256 tiles", flush=True)
+    ok(lib().uocr_hip_rswa_attention_ragged(ptr(dev_f32(q, dev)), ptr(dev_f32(K, dev)), ptr(dev_f32(V, dev)),
+                                            ptr(dev_i32(slots, dev)), ptr(dev_i32(pos, dev)), total, cap, heads,
+                                            kv_heads, hd, ptr(out), None))
+    torch.cuda.synchronize()
+    want = _rows_want(q, K, V, slots, pos, heads, kv_heads, hd)
+    assert np.abs(out.cpu().numpy().reshape(total, -1) - want).max() <= TOL

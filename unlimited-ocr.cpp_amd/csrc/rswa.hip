@@ -92,9 +92,8 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
 //     dims 4 i + b.
 // The rows of a tile may belong to several requests (slots): one pass over the
 // keys per distinct slot, rows of other slots masked. Where that costs more
-// than walking the rows one by one (a key block of a pass costs about four
-// row-blocks of the row kernel: 9 against 2.2 ns on the whole chip), the tile
-// is left to row workers, extra workgroups at the grid's end.
+// than walking the rows one by one (tile_pays), the tile is left to row
+// workers, extra workgroups at the grid's end.
 // Bound by the f32 MFMA rate (154 TFLOP/s on a large product; 35 us of the
 // call below), the start of a workgroup (9k cycles to its first scores) and the grid's end.
 // Measured (rocprofv3) at 4 requests of 358..1000 rows, 10 heads of 128: 711 us
@@ -104,11 +103,11 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
 // V rows in flight with Q in registers (spills).
 // ---------------------------------------------------------------------------
 constexpr int kTileQ = 32;        // query rows per tile
-constexpr int kTileWaves = 4;     // two workgroups per CU (head_dim 128: 80 KiB of LDS each)
+constexpr int kTileWaves = 4;
+constexpr int kTileResident = 2;  // workgroups per CU (registers; head_dim 128: 80 KiB of LDS each)
 constexpr int kTileSort = kTileWaves * 64;  // tiles that a call orders by their keys (one per thread)
 static_assert(kTileSort <= 256, "a tile's index has 8 bits of its sort key");
 constexpr int kTileCost = 4;      // row-blocks that a tile's key block costs
-constexpr int kRowWorkers = 512;  // at most
 
 // slot and key limit (rows attended, 0 past the end) of query row t
 __device__ __forceinline__ void row_limit(const RswaArgs& a, int rows, int t, int& slot, int& limit) {
@@ -132,43 +131,20 @@ __device__ __forceinline__ int half_max(int v) {  // over the 32 lanes of a half
     return v;
 }
 
-// whether a tile (lane l: row l % 32's slot and limit) runs as a tile;
-// wave-uniform. (Its buffer loads address up to 2 GiB of a request's cache.)
-__device__ __forceinline__ bool tile_size_ok(const RswaArgs& a, int limit) {
-    return (long long)limit * a.kv_heads * a.head_dim * 4 <= 0x7fffffffll;
-}
+// Whether a tile runs as a tile; every lane holds row l % 32's slot and limit, the
+// answer is that of its half wave's rows (a wave can ask about two tiles). Runs of rows
+// of one slot count as passes. (Its buffer loads address up to 2 GiB of a request's
+// cache.) A key block of a pass costs about four row-blocks of the row walk (9
+// against 2.2 ns on the whole chip).
 __device__ __forceinline__ bool tile_pays(const RswaArgs& a, int slot, int limit) {
-    if (!tile_size_ok(a, half_max(limit))) return false;
-    int rows = (limit + 31) / 32, cost = 0;
-    for (int o = 16; o >= 1; o >>= 1) rows += __shfl_xor(rows, o, 64);
-    uint32_t left = (uint32_t)__ballot(limit > 0);
-    while (left) {
-        const int s = __shfl(slot, __builtin_ctz(left), 64);
-        const bool in = slot == s && limit > 0;
-        cost += (half_max(in ? limit : 0) + 31) / 32 * kTileCost;
-        left &= ~(uint32_t)__ballot(in);
-    }
-    return __builtin_amdgcn_readfirstlane(cost) <= __builtin_amdgcn_readfirstlane(rows);
-}
-// by one thread: false if the tile certainly runs as a tile (its runs of rows of
-// one slot, an upper bound of its passes, cost no more than its rows)
-__device__ __forceinline__ bool tile_may_not_pay(const RswaArgs& a, int rows, int tile) {
-    int slots[kTileQ], limits[kTileQ];  // every load in flight before the first use
+    const int lane = threadIdx.x & 63, most = half_max(limit), most_blocks = (most + 31) / 32;
+    int blocks = (limit + 31) / 32;
 #pragma unroll
-    for (int r = 0; r < kTileQ; ++r) row_limit(a, rows, tile * kTileQ + r, slots[r], limits[r]);
-    int n = 0, cost = 0, run = 0, most = 0;
-#pragma unroll
-    for (int r = 0; r < kTileQ; ++r) {
-        const int blocks = (limits[r] + 31) / 32;
-        if (r > 0 && slots[r] != slots[r - 1]) {
-            cost += run;
-            run = 0;
-        }
-        run = max(run, blocks);
-        most = max(most, limits[r]);
-        n += blocks;
-    }
-    return !tile_size_ok(a, most) || (cost + run) * kTileCost > n;
+    for (int o = 16; o >= 1; o >>= 1) blocks += __shfl_xor(blocks, o, 64);
+    const int prev = __shfl_up(slot, 1, 32);
+    const bool first = slot >= 0 && ((lane & 31) == 0 || slot != prev);
+    const int runs = __popc((uint32_t)(__ballot(first) >> (lane & 32)));
+    return (long long)most * a.kv_heads * a.head_dim * 4 <= 0x7fffffffll && runs * most_blocks * kTileCost <= blocks;
 }
 
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
@@ -188,15 +164,16 @@ struct TileLds {
 };
 
 template <int HD>
-__global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs a, int rows, int n_tiles, bool sort) {
+__global__ __launch_bounds__(kTileWaves * 64, kTileResident) void rswa_tile_kernel(RswaArgs a, int rows, int n_tiles, bool sort) {
     constexpr int U = HD / 4;    // 16-byte units per row
     constexpr int NB = HD / 32;  // dims per lane of V, dim-blocks of O
     union Lds {
         TileLds<HD> t;
         RowLds<HD, kTileWaves> r;
         struct {
-            int list[kTileSort], n_list;
-        };
+            RowLds<HD, kTileWaves> r;
+            uint8_t pays[kTileSort];
+        } w;
         struct {
             __attribute__((aligned(16))) int pos[kTileSort];
             int tile;
@@ -208,28 +185,42 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
     const int i = lane & 31, h = lane >> 5;
     int slot, limit;
     if ((int)blockIdx.x >= n_tiles * a.heads) {  // row worker: the rows of the tiles that don't pay
-        const int w = blockIdx.x - n_tiles * a.heads, nw = gridDim.x - n_tiles * a.heads;
-        int& n_list = s.n_list;
+        // The rows of all such tiles, in order, go to the workers in turn: none is
+        // without a row while another has two more. us, restarting with worker 0 at
+        // every tile (320 of 512 had all the rows) / this / the row kernel: 10 heads of
+        // 128, requests of one row with 1000 keys: 128 289 / 220 / 219, 256 550 / 433 /
+        // 431; 100 requests of 3 rows 456 / 370 / 369.
+        int next = blockIdx.x - n_tiles * a.heads;  // this worker's next row, counted from tile t0 on
+        const int n_workers = gridDim.x - n_tiles * a.heads;
+        auto& c = s.w;
         for (int t0 = 0; t0 < n_tiles; t0 += kTileSort) {
-            if (tid == 0) n_list = 0;
-            __syncthreads();
-            if (t0 + tid < n_tiles && tile_may_not_pay(a, rows, t0 + tid)) s.list[atomicAdd(&n_list, 1)] = t0 + tid;
-            __syncthreads();
-            const int n_l = n_list, mine = tid < n_l ? s.list[tid] : 0;
-            __syncthreads();
-            for (int k = 0; k < n_l; ++k) {
-                if (tid == k) n_list = mine;
-                __syncthreads();
-                const int tile = n_list;
-                __syncthreads();  // (the rows' results take the list's place)
-                row_limit(a, rows, tile * kTileQ + i, slot, limit);
-                if (tile_pays(a, slot, limit)) continue;
-                const int n = min(kTileQ, rows - tile * kTileQ) * a.heads;
-                for (int j = w; j < n; j += nw) {
-                    row_attention<HD, kTileWaves>(a, tile * kTileQ + j / a.heads, j % a.heads, 0, s.r);
-                    __syncthreads();
+            const int n = min(kTileSort, n_tiles - t0);
+            for (int k0 = 0; k0 < n; k0 += 4 * 2 * kTileWaves) {  // one tile per half wave, four in flight
+                int sl[4], li[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) row_limit(a, rows, (t0 + k0 + j * 2 * kTileWaves + 2 * wave + h) * kTileQ + i, sl[j], li[j]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int k = k0 + j * 2 * kTileWaves + 2 * wave + h;
+                    const bool pays = tile_pays(a, sl[j], li[j]);
+                    if (i == 0 && k < n) c.pays[k] = pays;
                 }
             }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < kTileSort / 64; ++q) {
+                uint64_t left = __ballot(q * 64 + lane < n && !c.pays[q * 64 + lane]);
+                for (; left; left &= left - 1) {
+                    const int tile = t0 + q * 64 + __builtin_ctzll(left);
+                    const int m = min(kTileQ, rows - tile * kTileQ);
+                    for (; next < m * a.heads; next += n_workers) {
+                        row_attention<HD, kTileWaves>(a, tile * kTileQ + next / a.heads, next % a.heads, 0, c.r);
+                        __syncthreads();
+                    }
+                    next -= m * a.heads;
+                }
+            }
+            __syncthreads();  // (pays is read)
         }
         return;
     }
@@ -259,7 +250,7 @@ __global__ __launch_bounds__(kTileWaves * 64, 2) void rswa_tile_kernel(RswaArgs 
         __syncthreads();
     }
     row_limit(a, rows, tile * kTileQ + i, slot, limit);
-    if (!tile_pays(a, slot, limit)) return;
+    if (!__builtin_amdgcn_readfirstlane(tile_pays(a, slot, limit))) return;
     const int stride = a.kv_heads * HD;
     const int kvh = head / (a.heads / a.kv_heads);
     constexpr float kLog2e = 1.4426950408889634f;
@@ -571,6 +562,14 @@ std::mutex g_rswa_mu;
 float* g_rswa_part_ptr[64] = {};
 int g_rswa_cus[64] = {};
 
+int device_cus() {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        (void)hipGetLastError();
+    return n > 0 ? n : 256;
+}
+
 // device address of g_rswa_part and the CU count of the current device
 int rswa_device(float** part, int* cus) {
     int dev = 0;
@@ -613,8 +612,9 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
     // key split above)
     if (a.mode != 2 && rswa_call_tiled(rows, a.heads, a.head_dim, max_len)) {
         const int n_tiles = (rows + kTileQ - 1) / kTileQ;
-        const dim3 tgrid(n_tiles * a.heads + (int)std::min<long long>(wgs, kRowWorkers));
-        const bool sort = n_tiles * a.heads > 512;  // (two workgroups on each of 256 CUs)
+        const int resident = kTileResident * device_cus();  // workgroups that the chip holds at once
+        const dim3 tgrid(n_tiles * a.heads + (int)std::min<long long>(wgs, resident));
+        const bool sort = n_tiles * a.heads > resident;
         if (a.head_dim == 64) launch_k(rswa_tile_kernel<64>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
         else launch_k(rswa_tile_kernel<128>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
         const hipError_t te = hipGetLastError();
