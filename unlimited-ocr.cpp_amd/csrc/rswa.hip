@@ -134,9 +134,16 @@ __device__ __forceinline__ int half_max(int v) {  // over the 32 lanes of a half
 // Whether a tile runs as a tile; every lane holds row l % 32's slot and limit, the
 // answer is that of its half wave's rows (a wave can ask about two tiles). Runs of rows
 // of one slot count as passes. (Its buffer loads address up to 2 GiB of a request's
-// cache.) A key block of a pass costs about four row-blocks of the row walk (9
-// against 2.2 ns on the whole chip).
-__device__ __forceinline__ bool tile_pays(const RswaArgs& a, int slot, int limit) {
+// cache.) Two lines:
+//   * throughput: a key block of a pass costs about four row-blocks of the row walk (9
+//     against 2.2 ns on the whole chip);
+//   * time: the passes follow each other (7 us and 5.4 for each pass of short keys, 20
+//     more at 500 keys), while the call's rows are walked side by side (about 9 ns for each
+//     (row, head), 70 at 500 keys; 5.4 at head_dim 64). us, always tiled / by this
+//     rule / the row kernel: 30 requests of 4 rows 51 / 10.6 / 12.6, 16 of 10 28.1 / 12.9 /
+//     16.6, 100 of 10 29.9 / 29.1 / 93, 128 of 4 at 500 keys 193 / 192 / 371. A last tile
+//     with few rows has as little to walk (20 requests of 5 rows 11.8 / 9.7 / 10.5).
+__device__ __forceinline__ bool tile_pays(const RswaArgs& a, int rows, int slot, int limit) {
     const int lane = threadIdx.x & 63, most = half_max(limit), most_blocks = (most + 31) / 32;
     int blocks = (limit + 31) / 32;
 #pragma unroll
@@ -144,7 +151,11 @@ __device__ __forceinline__ bool tile_pays(const RswaArgs& a, int slot, int limit
     const int prev = __shfl_up(slot, 1, 32);
     const bool first = slot >= 0 && ((lane & 31) == 0 || slot != prev);
     const int runs = __popc((uint32_t)(__ballot(first) >> (lane & 32)));
-    return (long long)most * a.kv_heads * a.head_dim * 4 <= 0x7fffffffll && runs * most_blocks * kTileCost <= blocks;
+    const int live = __popc((uint32_t)(__ballot(slot >= 0) >> (lane & 32)));
+    return (long long)most * a.kv_heads * a.head_dim * 4 <= 0x7fffffffll && runs * most_blocks * kTileCost <= blocks &&
+           ((runs == 1 && live == kTileQ) ||
+            (runs + 1) * (most_blocks > 4 ? 300ll : a.head_dim == 64 ? 700ll : 600ll) * kTileQ <=
+                (long long)rows * a.heads * live);
 }
 
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
@@ -202,7 +213,7 @@ __global__ __launch_bounds__(kTileWaves * 64, kTileResident) void rswa_tile_kern
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int k = k0 + j * 2 * kTileWaves + 2 * wave + h;
-                    const bool pays = tile_pays(a, sl[j], li[j]);
+                    const bool pays = tile_pays(a, rows, sl[j], li[j]);
                     if (i == 0 && k < n) c.pays[k] = pays;
                 }
             }
@@ -250,7 +261,7 @@ __global__ __launch_bounds__(kTileWaves * 64, kTileResident) void rswa_tile_kern
         __syncthreads();
     }
     row_limit(a, rows, tile * kTileQ + i, slot, limit);
-    if (!__builtin_amdgcn_readfirstlane(tile_pays(a, slot, limit))) return;
+    if (!__builtin_amdgcn_readfirstlane(tile_pays(a, rows, slot, limit))) return;
     const int stride = a.kv_heads * HD;
     const int kvh = head / (a.heads / a.kv_heads);
     constexpr float kLog2e = 1.4426950408889634f;
