@@ -27,6 +27,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "rswa_dispatch.hpp"
+#include "xcd_order.hpp"
 #include "uocr_hip/moe_capi.h"
 
 namespace uocr_hip {
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
 // ---------------------------------------------------------------------------
 constexpr int kTileQ = 32;        // query rows per tile
 constexpr int kTileWaves = 4;
-constexpr int kTileResident = 2;  // workgroups per CU (registers; head_dim 128: 80 KiB of LDS each)
+constexpr int tile_resident(int head_dim) { return head_dim == 64 ? 3 : 2; }  // workgroups per CU (40 / 80 KiB of LDS each)
 constexpr int kTileSort = kTileWaves * 64;  // tiles that a call orders by their keys (one per thread)
 static_assert(kTileSort <= 256, "a tile's index has 8 bits of its sort key");
 constexpr int kTileCost = 4;      // row-blocks that a tile's key block costs
@@ -175,7 +176,7 @@ struct TileLds {
 };
 
 template <int HD>
-__global__ __launch_bounds__(kTileWaves * 64, kTileResident) void rswa_tile_kernel(RswaArgs a, int rows, int n_tiles, bool sort) {
+__global__ __launch_bounds__(kTileWaves * 64, tile_resident(HD)) void rswa_tile_kernel(RswaArgs a, int rows, int n_tiles, bool sort) {
     constexpr int U = HD / 4;    // 16-byte units per row
     constexpr int NB = HD / 32;  // dims per lane of V, dim-blocks of O
     union Lds {
@@ -223,9 +224,15 @@ __global__ __launch_bounds__(kTileWaves * 64, kTileResident) void rswa_tile_kern
                 uint64_t left = __ballot(q * 64 + lane < n && !c.pays[q * 64 + lane]);
                 for (; left; left &= left - 1) {
                     const int tile = t0 + q * 64 + __builtin_ctzll(left);
+                    // Grouped heads: 8 rows side by side, so that the heads of a row meet
+                    // in one XCD's L2 (200 requests of one row, 1000 keys, 8 / 2 heads of
+                    // 64: 133 -> 63 us). One head per KV head: the heads of a row side by
+                    // side, a whole row of the cache (128 requests, 10 heads of 128: 226 -> 220)
                     const int m = min(kTileQ, rows - tile * kTileQ);
+                    const int near = a.heads > a.kv_heads && m % kXcds == 0 ? kXcds : 1;
                     for (; next < m * a.heads; next += n_workers) {
-                        row_attention<HD, kTileWaves>(a, tile * kTileQ + next / a.heads, next % a.heads, 0, c.r);
+                        const int g = next / near;
+                        row_attention<HD, kTileWaves>(a, tile * kTileQ + g / a.heads * near + next % near, g % a.heads, 0, c.r);
                         __syncthreads();
                     }
                     next -= m * a.heads;
@@ -623,7 +630,7 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
     // key split above)
     if (a.mode != 2 && rswa_call_tiled(rows, a.heads, a.head_dim, max_len)) {
         const int n_tiles = (rows + kTileQ - 1) / kTileQ;
-        const int resident = kTileResident * device_cus();  // workgroups that the chip holds at once
+        const int resident = tile_resident(a.head_dim) * device_cus();  // workgroups that the chip holds at once
         const dim3 tgrid(n_tiles * a.heads + (int)std::min<long long>(wgs, resident));
         const bool sort = n_tiles * a.heads > resident;
         if (a.head_dim == 64) launch_k(rswa_tile_kernel<64>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
