@@ -33,3 +33,17 @@ def test_int4_tiles_zero_points(dev, seq, group, n_experts, top_k):
     L = awq_layer(seed=group, group=group, n_experts=n_experts, top_k=top_k, n_shared=1, hidden=hidden, inter=inter)
     x = synth.bf16_normal(np.random.default_rng(seq), (seq, hidden), 1.0)
     check_parity(L, x, dev, sample=16, label=f"int4 tile zeros g={group}")
+
+
+@pytest.mark.parametrize("seq,hidden,inter,n_experts,top_k", [
+    (400, 1280, 896, 64, 6), (300, 256, 256, 64, 6), (1024, 640, 256, 64, 6),
+])
+def test_int4_tiles_skewed(dev, seq, hidden, inter, n_experts, top_k):
+    """Popular experts own several tiles, others none: the live tiles are a small
+    part of the list's capacity."""
+    from uocr_hip import synth
+    L = synth.random_layer(seed=seq, hidden=hidden, inter=inter, n_experts=n_experts, top_k=top_k, n_shared=1, group=32,
+                           router_bias=synth.zipf_bias(n_experts) * 4)
+    x = synth.bf16_normal(np.random.default_rng(seq), (seq, hidden), 1.0)
+    x[:, 0] = 1.0
+    check_parity(L, x, dev, sample=16, label=f"int4 tile skew H={hidden} I={inter}")

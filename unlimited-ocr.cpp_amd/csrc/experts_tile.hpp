@@ -25,6 +25,7 @@
 // k-tile's operands requested at once instead of one k-step ahead: 53 -> 46.5 at 256.
 #pragma once
 #include "experts_prefill.hpp"
+#include "xcd_order.hpp"
 
 namespace uocr_hip {
 
@@ -41,7 +42,7 @@ struct Int4Tile {
 };
 
 template <int BM, bool GU, int GPT, bool ZP>
-__global__ __launch_bounds__(256, 2) void int4_tile_kernel(ExpertArgs a, int n_tiles) {
+__global__ __launch_bounds__(256, 2) void int4_tile_kernel(ExpertArgs a) {
     using T = Int4Tile<BM>;
     constexpr int JM = BM / 64, SA = T::a_stages;
     constexpr int DA = BM / 32;                    // activation DMAs per wave and k-tile
@@ -49,13 +50,14 @@ __global__ __launch_bounds__(256, 2) void int4_tile_kernel(ExpertArgs a, int n_t
     constexpr int NC = GU ? 64 : 128;              // output columns
     __shared__ __attribute__((aligned(16))) uint8_t smem[T::lds];
     const int n_nt = a.n_rows / NC;
-    // block b runs on XCD b % 8; an XCD gets a contiguous run of (tile, n-tile) items,
-    // so the n-tiles of one tile share its activation rows in that XCD's L2
-    const int per_xcd = (n_nt * n_tiles + 7) / 8;
-    const int item = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if ((int)blockIdx.x / 8 >= per_xcd || item >= n_nt * n_tiles) return;
-    const int tile = item % n_tiles, nt = item / n_tiles;
-    if (tile >= *a.n_tiles) return;
+    // an XCD takes an even run of the live (tile, n-tile) items, n-tiles fastest: those of
+    // one tile share its activation rows in that XCD's L2. (Runs over the list's
+    // capacity gave some XCDs mostly dead entries: the whole call, us, 1024 tokens at hidden
+    // 1792, inter 256 110 -> 94; tiles fastest: 597 tokens of the decoder 107.7 against 105.4)
+    const int n_live = *a.n_tiles, xcd = blockIdx.x % kXcds;
+    const int item = xcd_first_item(xcd, n_live * n_nt) + blockIdx.x / kXcds;
+    if (item >= xcd_first_item(xcd + 1, n_live * n_nt)) return;
+    const int tile = item / n_nt, nt = item % n_nt;
     const int4 ti = *reinterpret_cast<const int4*>(a.tile_info + 4 * tile);  // expert, first row, live rows, first slot
     const int e = ti.x, rows = ti.z, slot0 = ti.w;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -274,9 +276,9 @@ static hipError_t launch_int4_tile(const ExpertArgs& a, int max_tiles, hipStream
     auto go = [&](auto bm) {
         constexpr int BM = decltype(bm)::value;
         switch (a.group) {
-            case 32: launch_k((int4_tile_kernel<BM, GU, 4, ZP>), grid, dim3(256), 0, st, a, max_tiles); break;
-            case 64: launch_k((int4_tile_kernel<BM, GU, 2, ZP>), grid, dim3(256), 0, st, a, max_tiles); break;
-            case 128: launch_k((int4_tile_kernel<BM, GU, 1, ZP>), grid, dim3(256), 0, st, a, max_tiles); break;
+            case 32: launch_k((int4_tile_kernel<BM, GU, 4, ZP>), grid, dim3(256), 0, st, a); break;
+            case 64: launch_k((int4_tile_kernel<BM, GU, 2, ZP>), grid, dim3(256), 0, st, a); break;
+            case 128: launch_k((int4_tile_kernel<BM, GU, 1, ZP>), grid, dim3(256), 0, st, a); break;
             default: return hipErrorInvalidValue;
         }
         return hipGetLastError();
