@@ -267,7 +267,7 @@ int dense_to_f16(const uocr_hip_dense_matrix& m, uint16_t* dst, std::string* err
 }
 
 struct WsPlan {
-    size_t x16, ids, wts, counts, offsets, ntiles, slot_tok, slot_w, pos, tile_e, tile_m0, tile_info, act, y, total;
+    size_t x16, ids, wts, offsets, ntiles, slot_tok, slot_w, pos, tile_info, act, y, total;
     size_t lrank, chunk_count, chunk_base;
     size_t sact, sy;  // unquantised shared MLP: act [seq, s_inter] f16, y [seq, hidden] f32
     int slots, max_tiles, bm;
@@ -384,14 +384,11 @@ WsPlan plan(const uocr_hip_moe_layer* L, int seq) {
     p.x16 = take((size_t)seq * L->hidden * 2);
     p.ids = take((size_t)seq * L->top_k * 4);
     p.wts = take((size_t)seq * L->top_k * 4);
-    p.counts = take((size_t)Ev * 4);
     p.offsets = take((size_t)(Ev + 1) * 4);
     p.ntiles = take(4);
     p.slot_tok = take((size_t)p.slots * 4);
     p.slot_w = take((size_t)p.slots * 4);
     p.pos = take((size_t)seq * L->top_k * 4);
-    p.tile_e = take((size_t)p.max_tiles * 4);
-    p.tile_m0 = take((size_t)p.max_tiles * 4);
     p.tile_info = take((size_t)p.max_tiles * 16);
     // act / y: one row per slot (y: per entry), or per (group, token) when the
     // fused decode kernel may run (seq <= kFusedMaxSeq, any input dtype)
@@ -1004,13 +1001,10 @@ int uocr_hip_moe_layer_forward(const uocr_hip_moe_layer* L, const void* x, int x
     g.n_experts = L->n_experts;
     g.n_virtual = L->n_virtual;
     g.bm = p.bm;
-    g.counts = (int*)(ws + p.counts);
     g.offsets = (int*)(ws + p.offsets);
     g.slot_tok = (int*)(ws + p.slot_tok);
     g.slot_w = (float*)(ws + p.slot_w);
     g.pos = (int*)(ws + p.pos);
-    g.tile_e = (int*)(ws + p.tile_e);
-    g.tile_m0 = (int*)(ws + p.tile_m0);
     g.tile_info = (int*)(ws + p.tile_info);
     g.n_tiles = (int*)(ws + p.ntiles);
     g.lrank = (int*)(ws + p.lrank);
@@ -1089,10 +1083,6 @@ int uocr_hip_moe_layer_forward(const uocr_hip_moe_layer* L, const void* x, int x
     gu.group = L->group;
     gu.bm = p.bm;
     gu.slot_tok = g.slot_tok;
-    gu.counts = g.counts;
-    gu.offsets = g.offsets;
-    gu.tile_e = g.tile_e;
-    gu.tile_m0 = g.tile_m0;
     gu.tile_info = g.tile_info;
     gu.n_tiles = g.n_tiles;
     gu.act_out = (f16*)(ws + p.act);

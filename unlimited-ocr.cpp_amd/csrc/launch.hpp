@@ -52,13 +52,10 @@ struct GroupArgs {
     const float* weights;
     int seq, top_k, n_experts, n_virtual, bm;
     // grouped-slot outputs (fused layer path); any may be null
-    int* counts;     // [n_experts + n_virtual]
     int* offsets;    // [n_experts + n_virtual + 1]
     int* slot_tok;   // [slots]
     float* slot_w;   // [slots]
     int* pos;        // [seq * top_k] slot of entry (t, j)
-    int* tile_e;     // [max tiles]
-    int* tile_m0;    // [max tiles]
     int* tile_info;  // [max tiles][4]: e, m0, rows, first slot (16-byte aligned)
     int* n_tiles;    // [1]
     // reference [n_experts, cap] assignment tables (moe_router_topk mirror)
@@ -88,10 +85,6 @@ struct ExpertArgs {
     int group;
     int bm;                  // slots per m-tile of the tile list
     const int* slot_tok;
-    const int* counts;
-    const int* offsets;
-    const int* tile_e;
-    const int* tile_m0;
     const int* tile_info;    // [max tiles][4]: e, m0, rows, first slot
     const int* n_tiles;
     f16* act_out;            // gate/up: [slots, n_rows] f16
@@ -217,7 +210,7 @@ hipError_t launch_combine(const CombineArgs& c, hipStream_t st);
 // [experts][rows][cols] on the device (dense.hip).
 constexpr int kDenseSkinnyBM = 16;   // decode-sized tiles
 constexpr int kDenseTiledBM = 128;   // prefill-sized tiles
-constexpr int kDenseTiledSmallBM = 64;  // and the smaller ones of a short prefill (shared MLP)
+constexpr int kDenseTiledSmallBM = 64;  // and the smaller ones of a short prefill
 struct DenseArgs {
     const void* a;          // A rows: f16 (x16 / act) or bf16 (the layer input x)
     int a_kind;             // 0 f16, 1 bf16

@@ -138,11 +138,7 @@ __device__ __forceinline__ void write_tile_list(const GroupArgs& g, const int* h
     for (int e = wave; e < Ev; e += kGroupWaves) {
         const int nt = tile0[e + 1] - tile0[e];
         auto put = [&](int idx, int m0) {
-            g.tile_e[idx] = e;
-            g.tile_m0[idx] = m0;
-            if (g.tile_info)
-                *reinterpret_cast<int4*>(g.tile_info + 4 * idx) =
-                    make_int4(e, m0, min(g.bm, hist[e] - m0), offs[e] + m0);
+            *reinterpret_cast<int4*>(g.tile_info + 4 * idx) = make_int4(e, m0, min(g.bm, hist[e] - m0), offs[e] + m0);
         };
         for (int m = lane; m < nt; m += 64) put(tile0[e] + m, m * g.bm);
         if (lane == 0 && short0[e + 1] > short0[e]) put(nlong + short0[e], nt * g.bm);
@@ -170,7 +166,7 @@ __device__ void group_body(const int* ids, const float* wts, const GroupArgs& g,
     }
     __syncthreads();
     if (wave == 0) wave0_exclusive_scan(s.hist, s.offs, Ev);
-    if (wave == 1 && g.tile_e) {
+    if (wave == 1 && g.tile_info) {
         // tiles per expert into run[] (reset below), then scan into tile0[]
         for (int e = lane; e < Ev; e += 64) {
             s.run[e] = long_tiles(s.hist[e], g.bm);
@@ -178,17 +174,14 @@ __device__ void group_body(const int* ids, const float* wts, const GroupArgs& g,
         }
     }
     __syncthreads();
-    if (g.tile_e && wave == 1) wave0_exclusive_scan(s.run, s.tile0, Ev);
-    if (g.tile_e && wave == 2) wave0_exclusive_scan(s.nshort, s.short0, Ev);
+    if (g.tile_info && wave == 1) wave0_exclusive_scan(s.run, s.tile0, Ev);
+    if (g.tile_info && wave == 2) wave0_exclusive_scan(s.nshort, s.short0, Ev);
     __syncthreads();
-    if (g.counts) {
-        for (int e = tid; e < Ev; e += kGroupThreads) {
-            g.counts[e] = s.hist[e];
-            g.offsets[e] = s.offs[e];
-        }
+    if (g.offsets) {
+        for (int e = tid; e < Ev; e += kGroupThreads) g.offsets[e] = s.offs[e];
         if (tid == 0) g.offsets[Ev] = s.offs[Ev];
     }
-    if (g.tile_e) write_tile_list(g, s.hist, s.offs, s.tile0, s.short0, Ev);
+    if (g.tile_info) write_tile_list(g, s.hist, s.offs, s.tile0, s.short0, Ev);
     for (int e = tid; e < kMaxExperts; e += kGroupThreads) s.run[e] = 0;
     __syncthreads();
     // stable placement of the routed entries, kGroupThreads entries per round
@@ -307,7 +300,7 @@ __global__ __launch_bounds__(kGroupThreads) void group_scan_kernel(GroupArgs g, 
     extern __shared__ int cc[];  // [n_chunks][E] counts, then bases
     __shared__ int hist[kMaxExperts], offs[kMaxExperts + 1], ntl[kMaxExperts], tile0[kMaxExperts + 1];
     __shared__ int nsh[kMaxExperts], short0[kMaxExperts + 1];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = tid >> 6;
     const int E = g.n_experts, Ev = E + g.n_virtual;
     for (int k = tid; k < n_chunks * E; k += kGroupThreads) cc[k] = g.chunk_count[k];
     __syncthreads();
@@ -332,17 +325,14 @@ __global__ __launch_bounds__(kGroupThreads) void group_scan_kernel(GroupArgs g, 
     __syncthreads();
     for (int k = tid; k < n_chunks * E; k += kGroupThreads) g.chunk_base[k] = cc[k] + (g.slot_tok ? offs[k % E] : 0);
     for (int e = tid; e < Ev; e += kGroupThreads) {
-        if (g.counts) {
-            g.counts[e] = hist[e];
-            g.offsets[e] = offs[e];
-        }
+        if (g.offsets) g.offsets[e] = offs[e];
         if (g.assign_count && e < E) {
             g.assign_count[e] = min(hist[e], g.cap);
             if (hist[e] > g.cap) atomicOr(&g_router_overflow, 1);
         }
     }
-    if (tid == 0 && g.counts) g.offsets[Ev] = offs[Ev];
-    if (g.tile_e) write_tile_list(g, hist, offs, tile0, short0, Ev);
+    if (tid == 0 && g.offsets) g.offsets[Ev] = offs[Ev];
+    if (g.tile_info) write_tile_list(g, hist, offs, tile0, short0, Ev);
     // virtual (shared-expert) groups: every token, weight 1
     if (g.slot_tok)
         for (int v = 0; v < g.n_virtual; ++v)
@@ -392,8 +382,8 @@ __global__ __launch_bounds__(kGroupThreads) void group_scan_place_kernel(GroupAr
     }
     __syncthreads();
     if (wave == 0) wave0_exclusive_scan(hist, offs, Ev);
-    if (b == 0 && g.tile_e && wave == 1) wave0_exclusive_scan(ntl, tile0, Ev);
-    if (b == 0 && g.tile_e && wave == 2) wave0_exclusive_scan(nsh, short0, Ev);
+    if (b == 0 && g.tile_info && wave == 1) wave0_exclusive_scan(ntl, tile0, Ev);
+    if (b == 0 && g.tile_info && wave == 2) wave0_exclusive_scan(nsh, short0, Ev);
     __syncthreads();
     if (valid) {
         if (g.slot_tok) {  // the slot
@@ -411,17 +401,14 @@ __global__ __launch_bounds__(kGroupThreads) void group_scan_place_kernel(GroupAr
     }
     if (b == 0) {
         for (int e = tid; e < Ev; e += kGroupThreads) {
-            if (g.counts) {
-                g.counts[e] = hist[e];
-                g.offsets[e] = offs[e];
-            }
+            if (g.offsets) g.offsets[e] = offs[e];
             if (g.assign_count && e < E) {
                 g.assign_count[e] = min(hist[e], g.cap);
                 if (hist[e] > g.cap) atomicOr(&g_router_overflow, 1);
             }
         }
-        if (tid == 0 && g.counts) g.offsets[Ev] = offs[Ev];
-        if (g.tile_e) write_tile_list(g, hist, offs, tile0, short0, Ev);
+        if (tid == 0 && g.offsets) g.offsets[Ev] = offs[Ev];
+        if (g.tile_info) write_tile_list(g, hist, offs, tile0, short0, Ev);
     }
     // virtual (shared-expert) groups: every token, weight 1
     if (g.slot_tok)
