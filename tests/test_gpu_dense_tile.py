@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("seq,hidden,inter,n_shared", [
     (65, 1280, 128, 2), (128, 256, 896, 2), (129, 1280, 128, 14), (1023, 128, 128, 1), (1024, 384, 128, 3),
     (1025, 384, 128, 3), (1300, 1280, 128, 1), (3300, 1280, 128, 1),
+    (96, 1280, 128, 2), (97, 1280, 128, 2), (97, 640, 896, 2),  # the smallest batch on 64-slot tiles
 ])
 def test_shared_mlp_tiles(dev, seq, hidden, inter, n_shared):
     from uocr_hip import synth

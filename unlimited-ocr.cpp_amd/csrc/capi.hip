@@ -354,11 +354,12 @@ int int4_bm(const uocr_hip_moe_layer* L, int seq) {
     return prefill_big_ok(L->hidden, L->inter) ? kPrefillBigTileRows : kPrefillTileRows;
 }
 // ... and of the unquantised shared MLP (every token: a plain GEMM). Both
-// launches, us, 16-slot / 64-slot / 128-slot tiles at hidden 1280, width 1792: 64
-// tokens 20.8 / 22.2, 65 19.7 / 18.4, 127 26.4 / 18.4 / 29, 512 - / 19.8 / 29.2, 1024
-// - / 29.5 / 30.5, 2048 - / 57.2 / 48.7
+// launches, us, 16-slot / 64-slot / 128-slot tiles at hidden 1280, width 1792: 65
+// tokens 20.1 / 21.1, 80 20.9 / 21.5, 96 21.0 / 21.9 (whole call 90.8 / 91.5), 112
+// 27.0 / 22.5 (98.3 / 93.5: the 16-slot gate/up needs a second round), 512 - / 23.0 /
+// 34.2, 1024 - / 36.7 / 36.1, 2048 - / 59.0 / 54.1
 int dense_shared_bm(const uocr_hip_moe_layer* L, int seq) {
-    if (seq <= 64 || !dense_shapes_ok(L->hidden, L->s_inter, true, kDenseTiledBM) ||
+    if (seq <= 96 || !dense_shapes_ok(L->hidden, L->s_inter, true, kDenseTiledBM) ||
         !dense_shapes_ok(L->s_inter, L->hidden, false, kDenseTiledBM))
         return kDenseSkinnyBM;
     return seq <= 1024 ? kDenseTiledSmallBM : kDenseTiledBM;
