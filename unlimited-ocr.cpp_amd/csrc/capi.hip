@@ -273,12 +273,13 @@ struct WsPlan {
     int slots, max_tiles, bm;
 };
 
-// Prefill (LDS-tiled MFMA GEMM, 128-slot m-tiles) once experts see enough
-// tokens to fill its tiles; the decode kernels (16-slot tiles, weights streamed
-// once per tile) below that.
+// Prefill (LDS-tiled MFMA GEMM, m-tiles of 64 to 256 slots) once experts see
+// enough tokens to fill its tiles; the decode kernels (16-slot tiles, weights
+// streamed once per tile) below that. (The line was measured with 256-slot tiles.)
 constexpr int kPrefillMinSeq = 256;
 // one workgroup per token in the router up to this batch (the router matrix is
-// then read once per token from L2); larger batches share it through LDS
+// then read once per token from L2); larger batches with a bf16 router take 16
+// tokens per workgroup
 constexpr int kRouterDecodeMaxSeq = 64;
 
 // Decode path (per-token router, grouping-free expert passes) below
@@ -335,9 +336,10 @@ bool use_stream(const uocr_hip_moe_layer* L, int seq, int x_dtype) {
 
 // Tile rows of the unquantised expert kernels: decode-sized tiles below the
 // prefill threshold, from there (when the shapes allow) 64 or 128 slots. 64 up to
-// 56 rows per expert on average, where most experts fill one such tile: gate/up +
-// down, us, 64 / 128 slots at 64 experts, top-6: 256 tokens 106 / 116, 512 119 /
-// 131, 768 172 / 143, 1111 170 / 154, 2048 258 / 236.
+// 56 rows per expert on average, where most experts fill one such tile. Whole
+// calls, us, 64 / 128 slots at 64 experts, top-6, even routing: 256 tokens 121 / 129,
+// 512 141 / 141, 597 149 / 157, 768 195 / 165, 1111 192 / 180, 2048 285 / 263; Zipf
+// routing: 256 82 / 84, 512 106 / 106, 597 114 / 119, 768 128 / 124, 1111 160 / 150.
 int dense_experts_bm(const uocr_hip_moe_layer* L, int seq) {
     if (seq < kPrefillMinSeq || !dense_shapes_ok(L->hidden, L->inter, true, kDenseTiledBM) ||
         !dense_shapes_ok(L->inter, L->hidden, false, kDenseTiledBM))
@@ -346,9 +348,14 @@ int dense_experts_bm(const uocr_hip_moe_layer* L, int seq) {
 }
 // ... and of the INT4 expert kernels. 64 slots, two workgroups per CU, up to 56
 // rows per expert on average; above, 256 slots (experts of at most 128 rows in half
-// mode) for the shapes it is built for, else 128. Gate/up + down, us, 64 / 128 / 256 slots
-// at 64 experts, top-6, group 32: 256 tokens 75 / 91 / 101, 512 83 / 99 / 102, 768 120 /
-// 105 / 108, 1024 131 / 114 / 108, 2048 219 / 193 / 189, 4096 402 / 329 / 299.
+// mode) for the shapes it is built for, else 128. Whole calls, us, 64 / 128 / 256 slots
+// at 64 experts, top-6, group 32, even routing: 256 tokens 89 / 107 / 128, 512 105 / 112 /
+// 131, 597 112 / 120 / 133, 700 131 / 122 / 134, 768 144 / 123 / 135, 1024 158 / 135 / 139,
+// 2048 243 / 215 / 220, 4096 425 / 350 / 338; Zipf routing: 256 70 / 72 / 92, 400 83 / 85 /
+// 93, 512 94 / 87 / 97, 597 100 / 100 / 104, 768 117 / 109 / 110, 1024 136 / 130 / 129, 2048
+// 234 / 198 / 207, 4096 410 / 338 / 327. Group 128 with zeros and Zipf routing, 128 / 256: 600
+// 109 / 107, 700 115 / 113, 1024 140 / 135, 2048 209 / 215, 2600 263 / 256: neither of
+// the two is the better one at every size, group and routing.
 int int4_bm(const uocr_hip_moe_layer* L, int seq) {
     if ((long long)seq * L->top_k <= 56ll * L->n_experts) return kPrefillSmallTileRows;
     return prefill_big_ok(L->hidden, L->inter) ? kPrefillBigTileRows : kPrefillTileRows;
@@ -860,7 +867,7 @@ int uocr_hip_moe_layer_forward(const uocr_hip_moe_layer* L, const void* x, int x
         sa.seq = seq;
         sa.out16 = (f16*)(ws + p.sact);
         sa.status = &L->sync->error;
-        // the 128-slot tiles take f16 input only
+        // the tiles above 16 slots take f16 input only
         HIP_TRY(launch_dense(sa, true, kind == 0 ? bm : kDenseSkinnyBM, 0, st), "shared gate/up launch");
         DenseArgs sd{};
         sd.a = sa.out16;

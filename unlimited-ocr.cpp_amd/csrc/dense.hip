@@ -161,11 +161,13 @@ __global__ __launch_bounds__(64 * NW) void dense_skinny_kernel(DenseArgs a) {
 //     rows then cover all 64 banks;
 //   * the LDS reads are asm with counted waits (the compiler would wait for
 //     every DMA in flight before each of them).
-// Small batches are bound by latency (few workgroups, K / 64 dependent steps),
-// large ones by L2 and LDS reads. Measured against the older kernel (128 slots, one
+// Small batches are bound by latency (few workgroups, K / 64 dependent steps). 64
+// experts at 1111 tokens: HBM, gate/up 374 MB in 96 us (303 of weights), down 312 MB in 57
+// (5.4 TB/s; 151 of weights, every XCD reads all act rows); MFMA 21 and 17% of the time, LDS
+// 10 and 8%. Measured against the older kernel (128 slots, one
 // k-tile of operand-order DMA ahead, 42 and 15 workgroups at 283 tokens), both
-// launches of the shared MLP: 283 tokens 97 -> 19.4 us, 1024 99 -> 29.5, 4096
-// 141 -> 100.
+// launches of the shared MLP, weights from HBM: 283 tokens 102 -> 22 us, 1024 108 -> 37, 4096
+// 137 -> 93.
 // ---------------------------------------------------------------------------
 template <int BM, int NJ>
 struct DenseTile {

@@ -1,5 +1,5 @@
 // Asm loads, LDS accesses and counted waits of the tiled expert kernels, and
-// the large-tile INT4 expert GEMM of a large prefill (MFMA-bound). Work items are
+// the large-tile INT4 expert GEMM of a large prefill. Work items are
 // (m-tile of up to 256 grouped slots of one expert, n-tile) taken from the device
 // tile list, so skewed experts (Zipf routing) simply own more m-tiles; the fused
 // gate/up pass pairs gate rows with the same up rows so SiLU(g)*u is formed in

@@ -7,7 +7,7 @@
 // moe_grouped_down_int4 (src/kernels/cuda/moe_gemm_int4.cu:535-732), which
 // stages bf16 panels for mma.sync m16n8k16. Here:
 //   * activation rows (gathered through the slot -> token list) come by 16-byte
-//     DMA in k-tiles of 64 columns, 2 or 3 k-tiles ahead; 8 lanes read a row's 128
+//     DMA in k-tiles of 64 columns, 2 (128 slots) or 3 k-tiles ahead; 8 lanes read a row's 128
 //     contiguous bytes;
 //   * weights: each thread loads 2 units (16 bytes of nibbles and the row's
 //     scales) per 128 columns into registers, 1 .. 2 of those ahead, and
@@ -20,9 +20,9 @@
 // A workgroup's load and store phases run under the other workgroup's MFMAs
 // (the 256-slot kernel of experts_prefill.hpp has one workgroup per CU). Bound by
 // the k-tile's chain (barrier, LDS latency, 8 or 16 MFMAs, staging): about 2400
-// cycles per 64 columns for two workgroups. Measured at 283 tokens, 64 experts, top-6, group
-// 32: gate/up 50.4 -> 47 us, down 37.5 -> 29 against the 256-slot kernel; all of a
-// k-tile's operands requested at once instead of one k-step ahead: 53 -> 46.5 at 256.
+// cycles per 64 columns for two workgroups (counters, gate/up at 283 tokens: MFMA 17% of
+// the time, LDS 31%, 2.1 TB/s from HBM). Measured at 283 tokens, 64 experts, top-6, group
+// 32: gate/up 50.4 -> 42 us, down 37.5 -> 25.5 against the 256-slot kernel.
 #pragma once
 #include "experts_prefill.hpp"
 #include "xcd_order.hpp"

@@ -4,7 +4,7 @@
 // Bit-exactness contract with the reference CPU path:
 //   logits   src/kernels/cpu_ops.cpp:26-39 -- one sequential fmaf chain per
 //            (token, expert), k ascending (the -march=native build contracts
-//            `acc += x * w`); one lane per expert runs exactly that chain.
+//            `acc += x * w`); a chain of f32 MFMAs gives exactly those bits.
 //   rmsnorm  src/kernels/cpu_ops.cpp:58-67 -- as the reference's -O3
 //            -march=native build runs it: each x*x rounded, summed in column
 //            order (only a scalar tail of H % 4 terms would be fused),

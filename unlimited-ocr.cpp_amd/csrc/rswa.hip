@@ -95,8 +95,9 @@ __global__ __launch_bounds__(kRswaWaves * 64) void rswa_kernel(RswaArgs a) {
 // keys per distinct slot, rows of other slots masked. Where that costs more
 // than walking the rows one by one (tile_pays), the tile is left to row
 // workers, extra workgroups at the grid's end.
-// Bound by the f32 MFMA rate (154 TFLOP/s on a large product; 35 us of the
-// call below), the start of a workgroup (9k cycles to its first scores) and the grid's end.
+// Its parts: the f32 MFMAs (154 TFLOP/s on a large product: 35 us of the call
+// below; busy for 31% of the time by the counters), the masked half of the blocks on the
+// diagonal, the start of a workgroup (9k cycles to its first scores) and the grid's end.
 // Measured (rocprofv3) at 4 requests of 358..1000 rows, 10 heads of 128: 711 us
 // row by row, 123 us tiled; error against 64 bits 1.41e-7 both ways (one
 // chain per score and per output is 7% faster and 3.2e-7 off). Not kept: 8
