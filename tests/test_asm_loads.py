@@ -113,7 +113,7 @@ def in_flight_uses(ins, labels):
     return sorted(found.items())
 
 
-def test_checker_sees_a_register_reused_under_its_load():
+def test_a_register_reused_under_its_load_is_seen():
     ins = ["global_load_dword v1, v[2:3], off", "s_mov_b64 s[0:1], -1", "s_and_b64 vcc, exec, s[0:1]",
            "s_cbranch_vccnz .E", "v_mov_b32_e32 v1, 0", "v_mov_b32_e32 v4, 0", "s_waitcnt vmcnt(0)",
            "v_mov_b32_e32 v1, 0", "s_endpgm"]

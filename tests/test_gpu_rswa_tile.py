@@ -1,6 +1,8 @@
 """The query-tiled attention kernel (head_dim 64 or 128, 98304 or more (row,
-head, key) triples) against the oracle: tile and key-block edges, rows of several requests
-in one tile, tiles left to the row workers, grouped heads, empty rows.
+head, key) triples, 262144 at head_dim 64, with as many keys as the call has rows) against the
+oracle: tile and key-block edges, rows of several requests in one tile, tiles left to the row
+workers, grouped heads, empty rows. A last tile of few rows is left to the row workers too:
+calls of 32 n + 28 rows run it as a tile.
 
 Both kernels hold everything in f32; the tolerance is that of the row kernel's
 tests (1e-4 absolute on outputs of order 1)."""
@@ -20,7 +22,8 @@ def _torch():
 
 @pytest.mark.parametrize("hd,kv_heads,heads", [(128, 10, 10), (64, 2, 8), (128, 2, 6)])
 @pytest.mark.parametrize("lens", [
-    [260],                       # one request, a ragged last tile
+    [260],                       # one request, the last tile's 4 rows to the row workers
+    [284],                       # one request, a ragged last tile
     [31, 33, 64, 1, 129],        # tile boundaries inside and between requests
     [3] * 40 + [70],             # short requests: tiles of many slots
 ])
@@ -75,7 +78,8 @@ def test_ragged_rows_in_any_order(dev):
 
 
 @pytest.mark.parametrize("seq,q_start,kv_len,causal", [(64, 936, 1000, 1), (129, 0, 129, 1), (300, 0, 33, 0),
-                                                       (180, -120, 60, 1), (210, 0, 50, 1)])
+                                                       (180, -120, 60, 1), (210, 0, 50, 1),
+                                                       (220, 0, 60, 0), (252, -30, 222, 1)])  # ragged last tiles
 def test_one_cache_tiles(dev, seq, q_start, kv_len, causal):
     """The query-block entry points with the length on the host and on the
     device; rows before the first key (q_start < 0) have no keys and give 0."""
@@ -103,13 +107,14 @@ def test_one_cache_tiles(dev, seq, q_start, kv_len, causal):
         assert np.abs(out.cpu().numpy().reshape(seq, -1) - want).max() <= TOL, devlen
 
 
+@pytest.mark.parametrize("last", [33, 57])  # a last tile for the row workers, and one that runs as a tile
 @pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
-def test_keys_past_the_limit_are_not_used(dev, hd, heads, kv_heads):
+def test_keys_past_the_limit_are_not_used(dev, hd, heads, kv_heads, last):
     """Rows of the cache past each request's length hold NaN and inf: the last
     key block's tail must not reach the output (a weight of 0 times NaN would)."""
     torch = _torch()
     rng = np.random.default_rng(hd)
-    lens, cap = [97, 130, 33], 200
+    lens, cap = [97, 130, last], 200
     n = len(lens)
     K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
     for s, m in enumerate(lens):
@@ -132,13 +137,14 @@ def test_keys_past_the_limit_are_not_used(dev, hd, heads, kv_heads):
         t0 += m
 
 
+@pytest.mark.parametrize("last", [33, 57])  # a last tile for the row workers, and one that runs as a tile
 @pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
-def test_non_finite_values_stay_with_their_rows(dev, hd, heads, kv_heads):
+def test_non_finite_values_stay_with_their_rows(dev, hd, heads, kv_heads, last):
     """One request's V holds inf and NaN: the other requests' rows in the same
     tiles, and its own rows before those positions, don't see them."""
     torch = _torch()
     rng = np.random.default_rng(hd + 1)
-    lens, cap = [97, 130, 33], 200
+    lens, cap = [97, 130, last], 200
     n = len(lens)
     K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
     V[1, 70, :, 3], V[1, 100] = np.inf, np.nan
@@ -165,13 +171,14 @@ def test_non_finite_values_stay_with_their_rows(dev, hd, heads, kv_heads):
         t0 += m
 
 
+@pytest.mark.parametrize("last", [33, 49])
 @pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
-def test_output_may_be_the_queries(dev, hd, heads, kv_heads):
+def test_output_may_be_the_queries(dev, hd, heads, kv_heads, last):
     """out == q, with inf and NaN values in reach of some rows (whose tiles are
     partly done again): the same bits as with an output of its own."""
     torch = _torch()
     rng = np.random.default_rng(hd + 2)
-    lens, cap = [197, 230, 33], 300
+    lens, cap = [197, 230, last], 300
     n = len(lens)
     K, V = rand(rng, n, cap, kv_heads, hd), rand(rng, n, cap, kv_heads, hd)
     V[1, 70, :, 3], V[1, 100], K[0, 190] = np.inf, np.nan, np.nan
