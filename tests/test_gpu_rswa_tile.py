@@ -1,5 +1,5 @@
-"""The query-tiled attention kernel (head_dim 64 or 128, 98304 or more (row,
-head, key) triples, 262144 at head_dim 64, with as many keys as the call has rows) against the
+"""The query-tiled attention kernel (head_dim 64 or 128, 512 or more (row, head) pairs,
+where rswa_dispatch.hpp has the tiles faster than the rows) against the
 oracle: tile and key-block edges, rows of several requests in one tile, tiles left to the row
 workers, grouped heads, empty rows. A last tile of few rows is left to the row workers too:
 calls of 32 n + 28 rows run it as a tile.
@@ -217,6 +217,8 @@ def _rows_want(q, K, V, slots, pos, heads, kv_heads, hd):
 @pytest.mark.parametrize("name,lens,starts", [
     ("one row each", [1] * 203, "any"),                        # row workers only, more than one row each
     ("4 rows each", [4] * 60, 0), ("5 rows each", [5] * 45, 7),  # many passes: left to the workers
+    ("20 rows each at 130", [20] * 6, 130),                    # tiles of two requests, and of three left to the workers
+    ("52 rows at 100", [52, 53], 100),
     ("20 rows each", [20] * 14, 0),                            # few passes: tiles, a short last one
     ("mixed", [1] * 70 + [130, 1, 9, 64, 2], "any"),           # both kinds in one call
 ])

@@ -51,6 +51,7 @@ struct RswaArgs {
     int batch_cap;
     int n_chunks;  // > 1: keys split over blockIdx.z, partial (m, l, o) records to part
     float* part;   // [rows][heads][n_chunks][kRswaRec]
+    float pairs, kv_share;  // (tiles) rows * heads, kv_heads / heads
 };
 
 // one partial record: m, l, (pad), then o[head_dim]
@@ -138,15 +139,17 @@ __device__ __forceinline__ int half_max(int v) {  // over the 32 lanes of a half
 // of one slot count as passes. (Its buffer loads address up to 2 GiB of a request's
 // cache.) Two lines:
 //   * throughput: a key block of a pass costs about four row-blocks of the row walk (9
-//     against 2.2 ns on the whole chip);
-//   * time: the passes follow each other (7 us and 5.4 for each pass of short keys, 20
-//     more at 500 keys), while the call's rows are walked side by side (about 9 ns for each
-//     (row, head), 70 at 500 keys; 5.4 at head_dim 64). us, always tiled / by this
-//     rule / the row kernel: 30 requests of 4 rows 51 / 10.6 / 12.6, 16 of 10 28.1 / 12.9 /
-//     16.6, 100 of 10 29.9 / 29.1 / 93, 128 of 4 at 500 keys 193 / 192 / 371. A last tile
-//     with few rows has as little to walk (20 requests of 5 rows 11.8 / 9.7 / 10.5).
-__device__ __forceinline__ bool tile_pays(const RswaArgs& a, int rows, int slot, int limit) {
-    const int lane = threadIdx.x & 63, most = half_max(limit), most_blocks = (most + 31) / 32;
+//     against 2.2 ns on the whole chip). (Every pass at the tile's most keys; each at its own
+//     tiles more of the tiles where a long request ends, but the workers ask about
+//     every tile: 40 requests of 35..117 rows, 8 heads over 2 of 64, 24 us -> 28)
+//   * time (rswa_tile_ns, rswa_rows_ns): the passes follow each other while the call's rows
+//     are walked side by side. us, always tiled / by this rule / the row kernel, 10 heads
+//     of 128: 30 requests of 4 rows 51 / 10.6 / 12.6, 16 of 10 28.1 / 12.9 / 16.6, 100 of 10
+//     29.9 / 29.1 / 93, 6 of 20 at position 400 71 / 42 / 45, 2 of 60 at 300 40 / 25.7 / 34.5. A
+//     last tile with few rows has as little to walk (20 requests of 5 rows 11.8 / 9.7 / 10.5).
+template <int HD>
+__device__ __forceinline__ bool tile_pays(const RswaArgs& a, int slot, int limit) {
+    const int lane = threadIdx.x & 63, most = half_max(limit);
     int blocks = (limit + 31) / 32;
 #pragma unroll
     for (int o = 16; o >= 1; o >>= 1) blocks += __shfl_xor(blocks, o, 64);
@@ -154,10 +157,10 @@ __device__ __forceinline__ bool tile_pays(const RswaArgs& a, int rows, int slot,
     const bool first = slot >= 0 && ((lane & 31) == 0 || slot != prev);
     const int runs = __popc((uint32_t)(__ballot(first) >> (lane & 32)));
     const int live = __popc((uint32_t)(__ballot(slot >= 0) >> (lane & 32)));
-    return (long long)most * a.kv_heads * a.head_dim * 4 <= 0x7fffffffll && runs * most_blocks * kTileCost <= blocks &&
+    return (long long)most * a.kv_heads * HD * 4 <= 0x7fffffffll && runs * ((most + 31) / 32) * kTileCost <= blocks &&
            ((runs == 1 && live == kTileQ) ||
-            (runs + 1) * (most_blocks > 4 ? 300ll : a.head_dim == 64 ? 700ll : 600ll) * kTileQ <=
-                (long long)rows * a.heads * live);
+            rswa_tile_ns(HD, most, runs) * kTileQ <=
+                rswa_rows_ns(HD, a.pairs, live, 32 * blocks - 16 * live, min(runs - 1, 5) * a.kv_share));
 }
 
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
@@ -215,7 +218,7 @@ __global__ __launch_bounds__(kTileWaves * 64, tile_resident(HD)) void rswa_tile_
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int k = k0 + j * 2 * kTileWaves + 2 * wave + h;
-                    const bool pays = tile_pays(a, rows, sl[j], li[j]);
+                    const bool pays = tile_pays<HD>(a, sl[j], li[j]);
                     if (i == 0 && k < n) c.pays[k] = pays;
                 }
             }
@@ -269,7 +272,7 @@ __global__ __launch_bounds__(kTileWaves * 64, tile_resident(HD)) void rswa_tile_
         __syncthreads();
     }
     row_limit(a, rows, tile * kTileQ + i, slot, limit);
-    if (!__builtin_amdgcn_readfirstlane(tile_pays(a, rows, slot, limit))) return;
+    if (!__builtin_amdgcn_readfirstlane(tile_pays<HD>(a, slot, limit))) return;
     const int stride = a.kv_heads * HD;
     const int kvh = head / (a.heads / a.kv_heads);
     constexpr float kLog2e = 1.4426950408889634f;
@@ -629,11 +632,15 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
     }
     // One cache or ragged rows may run query-tiled (fewer than 512 pairs keep the
     // key split above)
-    if (a.mode != 2 && rswa_call_tiled(rows, a.heads, a.head_dim, max_len)) {
+    const bool tiled = a.mode == 0 ? rswa_one_cache_tiled(rows, a.heads, a.head_dim, a.kv_len, a.q_start, a.causal)
+                                   : a.mode != 2 && rswa_call_tiled(rows, a.heads, a.head_dim, max_len);
+    if (tiled) {
         const int n_tiles = (rows + kTileQ - 1) / kTileQ;
         const int resident = tile_resident(a.head_dim) * device_cus();  // workgroups that the chip holds at once
         const dim3 tgrid(n_tiles * a.heads + (int)std::min<long long>(wgs, resident));
         const bool sort = n_tiles * a.heads > resident;
+        a.pairs = (float)wgs;
+        a.kv_share = (float)a.kv_heads / a.heads;
         if (a.head_dim == 64) launch_k(rswa_tile_kernel<64>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
         else launch_k(rswa_tile_kernel<128>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
         const hipError_t te = hipGetLastError();
