@@ -52,6 +52,7 @@ struct RswaArgs {
     int n_chunks;  // > 1: keys split over blockIdx.z, partial (m, l, o) records to part
     float* part;   // [rows][heads][n_chunks][kRswaRec]
     float pairs, kv_share;  // (tiles) rows * heads, kv_heads / heads
+    bool full;  // (tiles) they take most of the chip
 };
 
 // one partial record: m, l, (pad), then o[head_dim]
@@ -128,10 +129,21 @@ __device__ __forceinline__ void row_limit(const RswaArgs& a, int rows, int t, in
     limit = max(limit, 0);
 }
 
-__device__ __forceinline__ int half_max(int v) {  // over the 32 lanes of a half wave
-#pragma unroll
-    for (int o = 16; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-    return v;
+// over the 32 lanes of a half wave: DPP within 16 lanes, one LDS exchange between them
+// (the row workers ask about every tile, five exchanges per value kept them 6 us)
+template <class Op>
+__device__ __forceinline__ int half_reduce(int v, Op op) {
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true));   // quad_perm 1, 0, 3, 2
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true));   // quad_perm 2, 3, 0, 1
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true));  // row_half_mirror
+    v = op(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true));  // row_mirror
+    return op(v, __shfl_xor(v, 16, 64));
+}
+__device__ __forceinline__ int half_max(int v) {
+    return half_reduce(v, [](int x, int y) { return max(x, y); });
+}
+__device__ __forceinline__ int half_sum(int v) {
+    return half_reduce(v, [](int x, int y) { return x + y; });
 }
 
 // Whether a tile runs as a tile; every lane holds row l % 32's slot and limit, the
@@ -139,27 +151,32 @@ __device__ __forceinline__ int half_max(int v) {  // over the 32 lanes of a half
 // of one slot count as passes. (Its buffer loads address up to 2 GiB of a request's
 // cache.) Two lines:
 //   * throughput: a key block of a pass costs about four row-blocks of the row walk (9
-//     against 2.2 ns on the whole chip). (Every pass at the tile's most keys; each at its own
-//     tiles more of the tiles where a long request ends, but the workers ask about
-//     every tile: 40 requests of 35..117 rows, 8 heads over 2 of 64, 24 us -> 28)
+//     against 2.2 ns on the whole chip). Passes are taken at the tile's most keys; where the
+//     tiles fill more than 9/16 of the chip, the first request's at its own: a tile where a
+//     long request ends then stays a tile, but a call with idle CUs is done earlier by the
+//     workers (us, one / own, 8 heads over 2 of 64: 8 requests of 150..500 rows 39 / 33, 4
+//     of 90..300 15 / 17.5)
 //   * time (rswa_tile_ns, rswa_rows_ns): the passes follow each other while the call's rows
 //     are walked side by side. us, always tiled / by this rule / the row kernel, 10 heads
 //     of 128: 30 requests of 4 rows 51 / 10.6 / 12.6, 16 of 10 28.1 / 12.9 / 16.6, 100 of 10
 //     29.9 / 29.1 / 93, 6 of 20 at position 400 71 / 42 / 45, 2 of 60 at 300 40 / 25.7 / 34.5. A
-//     last tile with few rows has as little to walk (20 requests of 5 rows 11.8 / 9.7 / 10.5).
+//     last tile with few rows of one request runs beside its other tiles, at the same time
+//     (359 rows, 16 heads of 64: 15.3, by the workers 17.9), unless the call is as short as
+//     the tile (20 requests of 5 rows 11.8 / 9.7 / 10.5).
 template <int HD>
 __device__ __forceinline__ bool tile_pays(const RswaArgs& a, int slot, int limit) {
-    const int lane = threadIdx.x & 63, most = half_max(limit);
-    int blocks = (limit + 31) / 32;
-#pragma unroll
-    for (int o = 16; o >= 1; o >>= 1) blocks += __shfl_xor(blocks, o, 64);
-    const int prev = __shfl_up(slot, 1, 32);
+    const int lane = threadIdx.x & 63;
+    const int slot0 = lane & 32 ? __builtin_amdgcn_readlane(slot, 32) : __builtin_amdgcn_readlane(slot, 0);
+    const int most0 = half_max(slot == slot0 ? limit : 0), most1 = half_max(slot == slot0 ? 0 : limit);
+    const int most = max(most0, most1), blocks = half_sum((limit + 31) / 32);
+    const int prev = __builtin_amdgcn_update_dpp(0, slot, 0x138, 0xf, 0xf, true);  // the lane before (wave_shr:1)
     const bool first = slot >= 0 && ((lane & 31) == 0 || slot != prev);
     const int runs = __popc((uint32_t)(__ballot(first) >> (lane & 32)));
     const int live = __popc((uint32_t)(__ballot(slot >= 0) >> (lane & 32)));
-    return (long long)most * a.kv_heads * HD * 4 <= 0x7fffffffll && runs * ((most + 31) / 32) * kTileCost <= blocks &&
+    const int passes = a.full ? (most0 + 31) / 32 + (runs - 1) * ((most1 + 31) / 32) : runs * ((most + 31) / 32);
+    return (long long)most * a.kv_heads * HD * 4 <= 0x7fffffffll && passes * kTileCost <= blocks &&
            ((runs == 1 && live == kTileQ) ||
-            rswa_tile_ns(HD, most, runs) * kTileQ <=
+            rswa_tile_ns(HD, most, runs) * (runs == 1 ? 1.25f * live : (float)kTileQ) <=
                 rswa_rows_ns(HD, a.pairs, live, 32 * blocks - 16 * live, min(runs - 1, 5) * a.kv_share));
 }
 
@@ -640,6 +657,7 @@ int launch_attention(RswaArgs a, int rows, hipStream_t st, int max_len) {
         const dim3 tgrid(n_tiles * a.heads + (int)std::min<long long>(wgs, resident));
         const bool sort = n_tiles * a.heads > resident;
         a.pairs = (float)wgs;
+        a.full = (long long)n_tiles * a.heads * 16 > 9ll * resident;
         a.kv_share = (float)a.kv_heads / a.heads;
         if (a.head_dim == 64) launch_k(rswa_tile_kernel<64>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
         else launch_k(rswa_tile_kernel<128>, tgrid, dim3(kTileWaves * 64), 0, st, a, rows, n_tiles, sort);
