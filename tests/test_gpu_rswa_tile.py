@@ -1,8 +1,7 @@
 """The query-tiled attention kernel (head_dim 64 or 128, 512 or more (row, head) pairs,
 where rswa_dispatch.hpp has the tiles faster than the rows) against the
 oracle: tile and key-block edges, rows of several requests in one tile, tiles left to the row
-workers, grouped heads, empty rows. A last tile of few rows is left to the row workers too:
-calls of 32 n + 28 rows run it as a tile.
+workers, grouped heads, empty rows.
 
 Both kernels hold everything in f32; the tolerance is that of the row kernel's
 tests (1e-4 absolute on outputs of order 1)."""
@@ -22,8 +21,8 @@ def _torch():
 
 @pytest.mark.parametrize("hd,kv_heads,heads", [(128, 10, 10), (64, 2, 8), (128, 2, 6)])
 @pytest.mark.parametrize("lens", [
-    [260],                       # one request, the last tile's 4 rows to the row workers
-    [284],                       # one request, a ragged last tile
+    [260],                       # one request, 4 rows in the last tile
+    [284],                       # ... and 28
     [31, 33, 64, 1, 129],        # tile boundaries inside and between requests
     [3] * 40 + [70],             # short requests: tiles of many slots
 ])
@@ -107,7 +106,7 @@ def test_one_cache_tiles(dev, seq, q_start, kv_len, causal):
         assert np.abs(out.cpu().numpy().reshape(seq, -1) - want).max() <= TOL, devlen
 
 
-@pytest.mark.parametrize("last", [33, 57])  # a last tile for the row workers, and one that runs as a tile
+@pytest.mark.parametrize("last", [33, 57])  # a last tile of 4 rows, for the row workers, and one of 28
 @pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
 def test_keys_past_the_limit_are_not_used(dev, hd, heads, kv_heads, last):
     """Rows of the cache past each request's length hold NaN and inf: the last
@@ -137,7 +136,7 @@ def test_keys_past_the_limit_are_not_used(dev, hd, heads, kv_heads, last):
         t0 += m
 
 
-@pytest.mark.parametrize("last", [33, 57])  # a last tile for the row workers, and one that runs as a tile
+@pytest.mark.parametrize("last", [33, 57])  # a last tile of 4 rows, for the row workers, and one of 28
 @pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
 def test_non_finite_values_stay_with_their_rows(dev, hd, heads, kv_heads, last):
     """One request's V holds inf and NaN: the other requests' rows in the same
@@ -213,11 +212,12 @@ def _rows_want(q, K, V, slots, pos, heads, kv_heads, hd):
     return out.reshape(T, -1)
 
 
-@pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2)])
+@pytest.mark.parametrize("hd,heads,kv_heads", [(128, 10, 10), (64, 8, 2), (128, 32, 8), (64, 32, 8)])
 @pytest.mark.parametrize("name,lens,starts", [
+    ("a long end", [129, 95, 65, 97, 80], 0),  # a tile with its last row: 32 heads fill the chip and keep it a tile
     ("one row each", [1] * 203, "any"),                        # row workers only, more than one row each
     ("4 rows each", [4] * 60, 0), ("5 rows each", [5] * 45, 7),  # many passes: left to the workers
-    ("20 rows each at 130", [20] * 6, 130),                    # tiles of two requests, and of three left to the workers
+    ("20 rows each at 130", [20] * 6, 130),                    # long keys, two or three requests in a tile: left to the workers
     ("52 rows at 100", [52, 53], 100),
     ("20 rows each", [20] * 14, 0),                            # few passes: tiles, a short last one
     ("mixed", [1] * 70 + [130, 1, 9, 64, 2], "any"),           # both kinds in one call
